@@ -93,6 +93,28 @@ constexpr int cdm_ntri = cdm::tri_size(NPARAMS);
 //                              Predicted_Signal_Cached and fills the analytic
 //                              entries of Partial_Derivatives_Cached from one
 //                              evaluation of the shared parts
+//   CDM_GRID_LINEAR b          GridSearch: the signal is a weighted sum of basis
+//                              signals, S = sum_k w_k B_k, and the parameters
+//                              in b enter the weights only
+//                              (Grid_Weights(npar, P, FixP, w), in double).
+//                              The basis is evaluated at two levels, the first
+//                              CDM_GRID_SHARED_BASIS signals and what else the
+//                              others need once per combination of the
+//                              parameters in CDM_GRID_SHARED (kept per
+//                              measurement: CDM_GRID_SHARED_VALUES values of
+//                              Grid_Shared, from which Grid_Shared_Basis reads
+//                              its signals), the other CDM_GRID_OUTER_BASIS
+//                              signals once per combination of all parameters
+//                              outside b (Grid_Outer_Basis).  Both read
+//                              CDM_GRID_COMMON values per measurement
+//                              (Grid_Common, once per block).  Scalars are
+//                              formed by Grid_Table (CDM_GRID_TABLE doubles that
+//                              depend on the parameters in
+//                              CDM_GRID_TABLE_DEPENDS alone, a subset of
+//                              CDM_GRID_SHARED), Grid_Frame (CDM_GRID_FRAME
+//                              values, parameters CDM_GRID_FRAME_DEPENDS, also
+//                              a subset) and Grid_Outer (CDM_GRID_OUTER values
+//                              per outer combination)
 // Without them the plug-in's Predicted_Signal / Partial_Derivatives are used.
 #ifdef CDM_VOXEL_CACHE
 constexpr int cdm_vc = CDM_VOXEL_CACHE;
@@ -452,13 +474,17 @@ __device__ __forceinline__ double cdm_gs_sumsq(const cdm_gs_args& a, const float
   return cdm::Group<L>::sum(sumsq);
 }
 
+// The FP32 error band above cost b0 (rounding of the forward model and of the
+// residual sum, generous by a factor ~10).
+__device__ __forceinline__ double cdm_gs_band(double b0, double sumsq) {
+  return 4e-5 * sqrt(fmax(b0, 0.0) * sumsq) + 1e-4 * b0 + 1e-8 * sumsq;
+}
+
 // Whether more than the K listed combinations may sit within the FP32 error
-// band of the best (rounding of the forward model and of the residual sum,
-// generous by a factor ~10): then every combination is rescored in FP64.
+// band of the best: then every combination is rescored in FP64.
 __device__ __forceinline__ bool cdm_gs_crowded(const cdm_gs_voxel& w, double sumsq) {
   const double b0 = w.best_c[0];
-  const double band = 4e-5 * sqrt(fmax(b0, 0.0) * sumsq) + 1e-4 * b0 + 1e-8 * sumsq;
-  return w.best_i[CDM_GS_TOPK - 1] >= 0 && (double)w.best_c[CDM_GS_TOPK - 1] <= b0 + band;
+  return w.best_i[CDM_GS_TOPK - 1] >= 0 && (double)w.best_c[CDM_GS_TOPK - 1] <= b0 + cdm_gs_band(b0, sumsq);
 }
 
 // FP64 cost of combination c.
@@ -726,6 +752,476 @@ __global__ void __launch_bounds__(cdm_block) cdm_gridsearch_pick_kernel(cdm_gs_a
   }
   cdm_gs_write(a, w, v, lane, bestd_i, bestd);
 }
+
+// ------------------------------------------- GridSearch over basis signals
+// For plug-ins that declare CDM_GRID_LINEAR.  A voxel's cost is a quadratic
+// form in the weights,
+//   SSE = y.y - 2 sum_k w_k (B_k.y) + sum_kl w_k w_l (B_k.B_l),
+// so the combinations that differ only in weight parameters cost a few
+// multiply-adds each once the products of their basis signals are summed over
+// the measurements, and what depends on CDM_GRID_SHARED only is evaluated once
+// for all combinations that share it.  The basis signals are evaluated in the
+// plug-in's precision (the signal's own arithmetic) and their products summed
+// in FP64, so the screened cost carries the rounding of the basis alone: its
+// error is no larger than the direct form's, which also rounds the weighted
+// sum and every residual (the quadratic form's own cancellation is about
+// 1e-14 y.y, against the error band's 1e-8 y.y).
+//
+// The screen keeps each voxel's least cost, its combination and the second
+// least cost.  When the second lies outside the FP32 error band of the least
+// (cdm_gs_band), the choice is settled: no other combination can be the FP64
+// argmin.  Otherwise the voxel goes on a list, and a second kernel scans its
+// combinations again and scores in FP64 those whose cost lies within the band
+// (cdm_gs_cost64, earliest combination on ties).
+//
+// Work split: L lanes per voxel over the measurements, as everywhere; the
+// shared values and the voxel's measurements sit in LDS, each lane reading
+// only the entries it wrote.  With L = 4 a combination's three or four sums
+// need two butterfly stages, and the combinations of the weight parameters are
+// spread over the lanes.
+//
+// Bound by VALU issue: about 18 slots per measurement and basis combination
+// (one exponential, the FP64 products).  Measured against the scan of every
+// combination: NODDI_Watson, 968 combinations, 99 measurements, 150k voxels
+// 90.1 -> 2.05 ms; Ball_2_Sticks, 729 combinations, 280 measurements, 50k voxels
+// 25.1 -> 1.45 ms; NODDI_Bingham, 11,050 combinations, 307 voxels 12.3 ->
+// 0.33 ms (the screen in 154 slices).  One loop over a row of adjacent values
+// and values staged per block, four measurements unrolled, against separate
+// arrays and the measurement cache read per combination: 3.53 -> 1.98 ms for
+// the Watson screen.
+#ifdef CDM_GRID_LINEAR
+constexpr bool cdm_gs_basis = sizeof(cdm_tf) != sizeof(double);
+constexpr unsigned cdm_gs_linear = CDM_GRID_LINEAR, cdm_gs_shared = CDM_GRID_SHARED;
+constexpr int cdm_gs_ns = CDM_GRID_SHARED_VALUES, cdm_gs_ks = CDM_GRID_SHARED_BASIS, cdm_gs_ko = CDM_GRID_OUTER_BASIS;
+constexpr int cdm_gs_nframe = CDM_GRID_FRAME, cdm_gs_nouter = CDM_GRID_OUTER, cdm_gs_nc = CDM_GRID_COMMON;
+constexpr int cdm_gs_nw = __builtin_popcount(cdm_gs_linear);  // weight parameters
+#ifdef CDM_GRID_TABLE
+constexpr int cdm_gs_ntab = CDM_GRID_TABLE;
+constexpr unsigned cdm_gs_table_dep = CDM_GRID_TABLE_DEPENDS;
+#else
+constexpr int cdm_gs_ntab = 0;
+constexpr unsigned cdm_gs_table_dep = 0;
+#endif
+constexpr unsigned cdm_gs_frame_dep = CDM_GRID_FRAME_DEPENDS;
+static_assert((cdm_gs_shared & cdm_gs_linear) == 0 && (cdm_gs_table_dep & ~cdm_gs_shared) == 0 &&
+                  (cdm_gs_frame_dep & ~cdm_gs_shared) == 0,
+              "grid parameter levels");
+#else
+constexpr bool cdm_gs_basis = false;
+constexpr unsigned cdm_gs_linear = 0, cdm_gs_shared = 0, cdm_gs_table_dep = 0, cdm_gs_frame_dep = 0;
+constexpr int cdm_gs_ntab = 0, cdm_gs_ns = 1, cdm_gs_nc = 0, cdm_gs_nw = 0;
+#endif
+constexpr int cdm_gs_row = cdm_gs_ns + 1;  // values per measurement of a voxel's LDS rows: Grid_Shared's, the measurement
+
+// The grid as a product: nshared combinations of the shared parameters, each
+// with nouter of the other basis parameters, each with ninner of the weight
+// parameters.  Position (sg * nouter + o) * ninner + j is combination
+// order[position].
+struct cdm_gs_plan {
+  int nshared, nouter, ninner;
+  unsigned grid;             // the grid's parameters
+  const float* outer_vals;   // [nshared * nouter][NP] grid values (of the first inner combination)
+  const float* inner_vals;   // [ninner][NP]
+  const int* order;          // [nshared * nouter * ninner]
+  int table_lds;             // Grid_Table's values of the block's shared combinations are in LDS
+  int table_fixed, frame_fixed;  // no grid parameter moves Grid_Table / Grid_Frame
+  int off_common, off_table, off_inner, off_rows;  // byte offsets in the dynamic LDS
+  int row_stride;            // values of a voxel's LDS rows
+};
+
+// What the screen hands on.  S slices of the shared combinations (S > 1:
+// each slice's result to part_*, [S][nvox], and the voxels' y.y to sumsq).
+// count, list, thr: the voxels to settle in FP64 and their thresholds;
+// rescan_*: [entry][SB] slice minima of the second scan.
+struct cdm_gs_work {
+  int S, SB;
+  float *part_c1, *part_c2;
+  int* part_i1;
+  double* sumsq;
+  int* count;
+  int* list;
+  double* thr;
+  double* rescan_c;
+  int* rescan_i;
+};
+
+__device__ __forceinline__ void cdm_gs_range(int n, int S, int z, int& b, int& e) {
+  b = (int)((long long)n * z / S);
+  e = (int)((long long)n * (z + 1) / S);
+}
+
+#ifdef CDM_GRID_LINEAR
+// Grid values of position o's outer combination over the voxel's own.
+__device__ __forceinline__ void cdm_gs_trial(const cdm_gs_plan& pl, int o, const float* base, cdm_tf* trial) {
+  const float* gv = pl.outer_vals + (size_t)o * cdm_np;
+#pragma unroll
+  for (int i = 0; i < cdm_np; ++i) trial[i] = (cdm_tf)(((pl.grid >> i) & 1u) ? gv[i] : base[i]);
+}
+
+// Block prologue after cdm_stage_cfp: the common values, the tables of shared
+// combinations [sg0, sg1) and the weight parameters' grid values.  Ends with a
+// barrier.
+__device__ __forceinline__ void cdm_gs_stage(const cdm_gs_args& a, const cdm_gs_plan& pl, const float* s_cfp,
+                                             const CDM_F64* s_mc, char* lds, int sg0, int sg1) {
+  cdm_tf* s_common = reinterpret_cast<cdm_tf*>(lds + pl.off_common);
+  for (int m = threadIdx.x; m < a.g.nmeas; m += blockDim.x) {
+    cdm_cfp_row<cdm_tf> crow;
+    Grid_Common(cdm_np, crow.at(s_cfp, m, a.g.cfp_ts), cdm_mc_row(s_mc, m), s_common + m * cdm_gs_nc);
+  }
+  float* s_inner = reinterpret_cast<float*>(lds + pl.off_inner);
+  for (int j = threadIdx.x; j < pl.ninner; j += blockDim.x) {
+    int k = 0;
+#pragma unroll
+    for (int i = 0; i < cdm_np; ++i)
+      if ((cdm_gs_linear >> i) & 1u) s_inner[j * cdm_gs_nw + k++] = pl.inner_vals[(size_t)j * cdm_np + i];
+  }
+#ifdef CDM_GRID_TABLE
+  if (pl.table_lds) {
+    CDM_F64* s_tab = reinterpret_cast<CDM_F64*>(lds + pl.off_table);
+    float zero[cdm_np];
+#pragma unroll
+    for (int i = 0; i < cdm_np; ++i) zero[i] = 0.f;
+    for (int sg = sg0 + threadIdx.x; sg < sg1; sg += blockDim.x) {
+      cdm_tf trial[cdm_np];
+      cdm_gs_trial(pl, sg * pl.nouter, zero, trial);
+      CDM_F64 tb[cdm_gs_ntab];
+      Grid_Table(cdm_np, trial, tb);
+#pragma unroll
+      for (int k = 0; k < cdm_gs_ntab; ++k) s_tab[(sg - sg0) * cdm_gs_ntab + k] = tb[k];
+    }
+  }
+#endif
+  __syncthreads();
+}
+
+// Costs of every combination of shared groups [sg0, sg1) (tables staged from
+// tab0 on), handed to take(position, cost, active) by all lanes of the group
+// together, lane j the weight combination j, j + L, ...  `rows`: the voxel's
+// LDS rows [nmeas][cdm_gs_row], its measurements in place.
+template <int L, class F>
+__device__ __forceinline__ void cdm_gs_scan(const cdm_gs_args& a, const cdm_gs_plan& pl, const float* s_cfp,
+                                            const CDM_F64* s_mc, const char* lds, cdm_tf* rows, cdm_gs_voxel& w,
+                                            double sumsq, int sg0, int sg1, int tab0, int lane, F take) {
+  constexpr int KS = cdm_gs_ks, KO = cdm_gs_ko, K = KS + KO, NT = cdm_gs_ntab > 0 ? cdm_gs_ntab : 1;
+  constexpr int R = cdm_gs_row;
+  const int M = a.g.nmeas;
+  const CDM_F64* s_tab = reinterpret_cast<const CDM_F64*>(lds + pl.off_table);
+  const float* s_inner = reinterpret_cast<const float*>(lds + pl.off_inner);
+  const cdm_tf* s_common = reinterpret_cast<const cdm_tf*>(lds + pl.off_common);
+  cdm_cfp_row<cdm_tf> crow;
+  cdm_tf sf[cdm_gs_nframe > 0 ? cdm_gs_nframe : 1];
+  CDM_F64 tb[NT];
+  CDM_F64 fxd[cdm_fixp_max], P[cdm_np];
+#pragma unroll
+  for (int k = 0; k < cdm_fixp_max; ++k) fxd[k] = (double)w.fx[k];
+#pragma unroll
+  for (int i = 0; i < cdm_np; ++i) P[i] = (double)w.base[i];
+  for (int sg = sg0; sg < sg1; ++sg) {
+    cdm_tf trial[cdm_np];
+    cdm_gs_trial(pl, sg * pl.nouter, w.base, trial);
+#ifdef CDM_GRID_TABLE
+    if (pl.table_lds) {
+#pragma unroll
+      for (int k = 0; k < NT; ++k) tb[k] = s_tab[(sg - tab0) * NT + k];
+    } else if (!pl.table_fixed || sg == sg0) {
+      Grid_Table(cdm_np, trial, tb);
+    }
+#endif
+    if (!pl.frame_fixed || sg == sg0) Grid_Frame(cdm_np, trial, sf);
+    double ys[KS], gs[KS * (KS + 1) / 2];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) ys[k] = 0.0;
+#pragma unroll
+    for (int k = 0; k < KS * (KS + 1) / 2; ++k) gs[k] = 0.0;
+    for (int m = lane; m < M; m += L) {
+      cdm_tf sh[cdm_gs_ns], bs[KS];
+      Grid_Shared(cdm_np, trial, crow.at(s_cfp, m, a.g.cfp_ts), w.fx, tb, sf, cdm_mc_row(s_mc, m), sh);
+#pragma unroll
+      for (int k = 0; k < cdm_gs_ns; ++k) rows[m * R + k] = sh[k];
+      Grid_Shared_Basis(cdm_np, sh, s_common + m * cdm_gs_nc, bs);
+      const double y = (double)rows[m * R + cdm_gs_ns];
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        ys[k] = fma((double)bs[k], y, ys[k]);
+#pragma unroll
+        for (int l = 0; l <= k; ++l) gs[k * (k + 1) / 2 + l] = fma((double)bs[k], (double)bs[l], gs[k * (k + 1) / 2 + l]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < KS; ++k) ys[k] = cdm::Group<L>::sum(ys[k]);
+#pragma unroll
+    for (int k = 0; k < KS * (KS + 1) / 2; ++k) gs[k] = cdm::Group<L>::sum(gs[k]);
+    for (int o = 0; o < pl.nouter; ++o) {
+      const int op = sg * pl.nouter + o;
+      cdm_gs_trial(pl, op, w.base, trial);
+      cdm_tf so[cdm_gs_nouter];
+      Grid_Outer(cdm_np, trial, tb, so);
+      double yo[KO], go[KO][K];
+#pragma unroll
+      for (int k = 0; k < KO; ++k) {
+        yo[k] = 0.0;
+#pragma unroll
+        for (int l = 0; l < K; ++l) go[k][l] = 0.0;
+      }
+#pragma unroll 4
+      for (int m = lane; m < M; m += L) {
+        const cdm_tf* cm = s_common + m * cdm_gs_nc;
+        cdm_tf sh[cdm_gs_ns], b[K];
+#pragma unroll
+        for (int k = 0; k < cdm_gs_ns; ++k) sh[k] = rows[m * R + k];
+        const double y = (double)rows[m * R + cdm_gs_ns];
+        Grid_Shared_Basis(cdm_np, sh, cm, b);
+        Grid_Outer_Basis(cdm_np, trial, cm, so, sh, b + KS);
+#pragma unroll
+        for (int k = 0; k < KO; ++k) {
+          const double bk = (double)b[KS + k];
+          yo[k] = fma(bk, y, yo[k]);
+#pragma unroll
+          for (int l = 0; l <= KS + k; ++l) go[k][l] = fma(bk, (double)b[l], go[k][l]);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < KO; ++k) {
+        yo[k] = cdm::Group<L>::sum(yo[k]);
+#pragma unroll
+        for (int l = 0; l <= KS + k; ++l) go[k][l] = cdm::Group<L>::sum(go[k][l]);
+      }
+      for (int j0 = 0; j0 < pl.ninner; j0 += L) {
+        const int j = j0 + lane;
+        const bool active = j < pl.ninner;
+        const int jj = active ? j : 0;
+        CDM_F64 wt[K], Pw[cdm_np];
+        int q = 0;
+#pragma unroll
+        for (int i = 0; i < cdm_np; ++i) {
+          Pw[i] = P[i];
+          if ((cdm_gs_linear >> i) & 1u) {
+            const double val = (double)s_inner[jj * cdm_gs_nw + q++];
+            if ((pl.grid >> i) & 1u) Pw[i] = val;
+          }
+        }
+        Grid_Weights(cdm_np, Pw, fxd, wt);
+        double cost = sumsq;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          double t = k < KS ? -2.0 * ys[k < KS ? k : 0] : -2.0 * yo[k >= KS ? k - KS : 0];
+#pragma unroll
+          for (int l = 0; l < k; ++l)
+            t = fma(2.0 * wt[l], k < KS ? gs[k < KS ? k * (k + 1) / 2 + l : 0] : go[k >= KS ? k - KS : 0][l], t);
+          t = fma(wt[k], k < KS ? gs[k < KS ? k * (k + 1) / 2 + k : 0] : go[k >= KS ? k - KS : 0][k], t);
+          cost = fma(wt[k], t, cost);
+        }
+        take(op * pl.ninner + jj, (float)cost, active);
+      }
+    }
+  }
+}
+
+// The voxel's measurements into its LDS row, and y.y.
+template <int L>
+__device__ __forceinline__ double cdm_gs_load_y(const cdm_gs_args& a, const float* mv, cdm_tf* rows, int lane) {
+  double s = 0.0;
+  for (int m = lane; m < a.g.nmeas; m += L) {
+    const float y = mv[m];
+    rows[m * cdm_gs_row + cdm_gs_ns] = y;
+    s = fma((double)y, (double)y, s);
+  }
+  return cdm::Group<L>::sum(s);
+}
+
+// (c1, i1, c2): the least cost, its position and the second least cost.
+struct cdm_gs_best {
+  float c1, c2;
+  int i1;
+  __device__ __forceinline__ void clear() {
+    c1 = c2 = INFINITY;
+    i1 = INT_MAX;
+  }
+  // A NaN or infinite cost changes nothing; c1 <= c2, so the new second is the
+  // median of the three.
+  __device__ __forceinline__ void add(float c, int i) {
+    c = fminf(c, INFINITY);
+    c2 = __builtin_amdgcn_fmed3f(c1, c2, c);
+    i1 = c < c1 ? i : i1;
+    c1 = fminf(c1, c);
+  }
+  __device__ __forceinline__ void merge(float o1, int oi, float o2) {
+    c2 = fminf(fmaxf(c1, o1), fminf(c2, o2));
+    if (o1 < c1 || (o1 == c1 && oi < i1)) {
+      c1 = o1;
+      i1 = oi;
+    }
+  }
+  template <int STAGE>
+  __device__ __forceinline__ void stage() {
+    merge(cdm::exchange<STAGE>(c1), cdm::exchange<STAGE>(i1), cdm::exchange<STAGE>(c2));
+  }
+  template <int L>
+  __device__ __forceinline__ void reduce() {
+    if constexpr (L >= 4) {
+      stage<1>();
+      stage<2>();
+    }
+    if constexpr (L >= 16) {
+      stage<4>();
+      stage<8>();
+    }
+    if constexpr (L >= 64) {
+      stage<16>();
+      stage<32>();
+    }
+  }
+};
+
+// The screened voxel's outputs when its choice is settled, an entry of the
+// list otherwise (and for the --debug voxel, whose record holds the FP64
+// cost).
+__device__ __forceinline__ void cdm_gs_settle(const cdm_gs_args& a, const cdm_gs_plan& pl, const cdm_gs_work& wk,
+                                              const cdm_gs_voxel& w, const cdm_gs_best& best, double sumsq, int v,
+                                              int lane) {
+  if (lane != 0) return;
+  if (best.i1 == INT_MAX) {
+    cdm_gs_write(a, w, v, 0, -1, 0.0);
+    return;
+  }
+  const double thr = (double)best.c1 + cdm_gs_band((double)best.c1, sumsq);
+  if ((double)best.c2 > thr && !(a.c.dbg && v == a.c.dbg_voxel)) {
+    cdm_gs_write(a, w, v, 0, pl.order[best.i1], (double)best.c1);
+    return;
+  }
+  const int e = atomicAdd(wk.count, 1);
+  wk.list[e] = v;
+  wk.thr[e] = thr;
+}
+
+// The screen: block (x, z) scans slice z of its voxels' shared combinations.
+template <int L>
+__global__ void __launch_bounds__(cdm_block) cdm_gs_basis_kernel(cdm_gs_args a, cdm_gs_plan pl, cdm_gs_work wk) {
+  extern __shared__ float s_cfp[];
+  char* lds = reinterpret_cast<char*>(s_cfp);
+  const CDM_F64* s_mc = cdm_stage_cfp(a.g, s_cfp);
+  int sg0, sg1;
+  cdm_gs_range(pl.nshared, wk.S, blockIdx.y, sg0, sg1);
+  cdm_gs_stage(a, pl, s_cfp, s_mc, lds, sg0, sg1);
+  const int v = blockIdx.x * (cdm_block / L) + threadIdx.x / L;
+  const int lane = threadIdx.x % L;
+  if (v >= a.g.nvox) return;
+  cdm_tf* rows = reinterpret_cast<cdm_tf*>(lds + pl.off_rows) + (size_t)(threadIdx.x / L) * pl.row_stride;
+  cdm_gs_voxel w;
+  cdm_gs_best best;
+  best.clear();
+  double sumsq = 0.0;
+  if (cdm_gs_begin(a, v, w)) {
+    sumsq = cdm_gs_load_y<L>(a, a.g.meas + (size_t)v * a.g.nmeas, rows, lane);
+    cdm_gs_scan<L>(a, pl, s_cfp, s_mc, lds, rows, w, sumsq, sg0, sg1, sg0, lane, [&](int i, float c, bool active) {
+      best.add(active ? c : INFINITY, i);
+    });
+    best.reduce<L>();
+  }
+  if (wk.S == 1) {
+    cdm_gs_settle(a, pl, wk, w, best, sumsq, v, lane);
+  } else if (lane == 0) {
+    const size_t o = (size_t)blockIdx.y * a.g.nvox + v;
+    wk.part_c1[o] = best.c1;
+    wk.part_c2[o] = best.c2;
+    wk.part_i1[o] = best.i1;
+    if (blockIdx.y == 0) wk.sumsq[v] = sumsq;
+  }
+}
+
+// The slices' results merged, 16 lanes per voxel.
+constexpr int cdm_gs_merge_lanes = 16;
+__global__ void __launch_bounds__(cdm_block) cdm_gs_basis_merge_kernel(cdm_gs_args a, cdm_gs_plan pl, cdm_gs_work wk) {
+  const int v = blockIdx.x * (cdm_block / cdm_gs_merge_lanes) + threadIdx.x / cdm_gs_merge_lanes;
+  const int lane = threadIdx.x % cdm_gs_merge_lanes;
+  if (v >= a.g.nvox) return;
+  cdm_gs_voxel w;
+  (void)cdm_gs_begin(a, v, w);
+  cdm_gs_best best;
+  best.clear();
+  for (int z = lane; z < wk.S; z += cdm_gs_merge_lanes) {
+    const size_t o = (size_t)z * a.g.nvox + v;
+    best.merge(wk.part_c1[o], wk.part_i1[o], wk.part_c2[o]);
+  }
+  best.reduce<cdm_gs_merge_lanes>();
+  cdm_gs_settle(a, pl, wk, w, best, wk.sumsq[v], v, lane);
+}
+
+// The listed voxels, SB slices each: the combinations within the band scored
+// in FP64 by the whole group, the slice's least (earliest on ties) stored.
+template <int L>
+__global__ void __launch_bounds__(cdm_block) cdm_gs_basis_rescan_kernel(cdm_gs_args a, cdm_gs_plan pl, cdm_gs_work wk) {
+  extern __shared__ float s_cfp[];
+  const int count = *wk.count;
+  constexpr int per = cdm_block / L;
+  const long long tasks = (long long)((count + per - 1) / per) * wk.SB;
+  if ((long long)blockIdx.x >= tasks) return;  // uniform over the block
+  char* lds = reinterpret_cast<char*>(s_cfp);
+  const CDM_F64* s_mc = cdm_stage_cfp(a.g, s_cfp);
+  cdm_gs_stage(a, pl, s_cfp, s_mc, lds, 0, pl.nshared);
+  const int lane = threadIdx.x % L;
+  cdm_tf* rows = reinterpret_cast<cdm_tf*>(lds + pl.off_rows) + (size_t)(threadIdx.x / L) * pl.row_stride;
+  for (long long t = blockIdx.x; t < tasks; t += gridDim.x) {
+    const int e = (int)(t / wk.SB) * per + threadIdx.x / L, z = (int)(t % wk.SB);
+    if (e >= count) continue;
+    const int v = wk.list[e];
+    const double thr = wk.thr[e];
+    const float* mv = a.g.meas + (size_t)v * a.g.nmeas;
+    cdm_gs_voxel w;
+    (void)cdm_gs_begin(a, v, w);
+    int sg0, sg1;
+    cdm_gs_range(pl.nshared, wk.SB, z, sg0, sg1);
+    const double sumsq = cdm_gs_load_y<L>(a, mv, rows, lane);
+    double bestd = INFINITY;
+    int besti = INT_MAX;
+    cdm_gs_scan<L>(a, pl, s_cfp, s_mc, lds, rows, w, sumsq, sg0, sg1, 0, lane, [&](int i, float c, bool active) {
+      const unsigned long long hits = __ballot(active && (double)c <= thr);
+      const int base = (int)(__lane_id() & ~(unsigned)(L - 1));
+      unsigned long long mine = L == 64 ? hits : (hits >> base) & ((1ull << (L & 63)) - 1);
+      while (mine) {
+        const int src = __ffsll(mine) - 1;
+        mine &= mine - 1;
+        const int comb = pl.order[cdm::Group<L>::bcast(i, src)];
+        const double cd = cdm_gs_cost64<L>(a, s_cfp, s_mc, mv, w, comb, lane);
+        if (cd < bestd || (cd == bestd && comb < besti)) {
+          bestd = cd;
+          besti = comb;
+        }
+      }
+    });
+    if (lane == 0) {
+      wk.rescan_c[(size_t)e * wk.SB + z] = bestd;
+      wk.rescan_i[(size_t)e * wk.SB + z] = besti;
+    }
+  }
+}
+
+// The listed voxels' outputs: the least of their slices, earliest on ties.
+// 16 lanes per entry.
+__global__ void __launch_bounds__(cdm_block) cdm_gs_basis_pick_kernel(cdm_gs_args a, cdm_gs_work wk) {
+  constexpr int L = cdm_gs_merge_lanes, per = cdm_block / L;
+  const int count = *wk.count, lane = threadIdx.x % L;
+  for (int e = blockIdx.x * per + threadIdx.x / L; e < count; e += gridDim.x * per) {
+    double bestd = INFINITY;
+    int besti = INT_MAX;
+    auto take = [&](double cd, int ci) {
+      if (cd < bestd || (cd == bestd && ci < besti)) {
+        bestd = cd;
+        besti = ci;
+      }
+    };
+    for (int z = lane; z < wk.SB; z += L) take(wk.rescan_c[(size_t)e * wk.SB + z], wk.rescan_i[(size_t)e * wk.SB + z]);
+    take(cdm::exchange<1>(bestd), cdm::exchange<1>(besti));
+    take(cdm::exchange<2>(bestd), cdm::exchange<2>(besti));
+    take(cdm::exchange<4>(bestd), cdm::exchange<4>(besti));
+    take(cdm::exchange<8>(bestd), cdm::exchange<8>(besti));
+    const int v = wk.list[e];
+    cdm_gs_voxel w;
+    (void)cdm_gs_begin(a, v, w);
+    cdm_gs_write(a, w, v, lane, besti == INT_MAX ? -1 : besti, bestd);
+  }
+}
+#endif  // CDM_GRID_LINEAR
 
 // ------------------------------------------------------ Levenberg-Marquardt
 // Levenberg_Marquardt.cu:409-623, with the bound transforms of :37-135 in

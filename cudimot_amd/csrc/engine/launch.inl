@@ -69,6 +69,108 @@ static hipError_t op_gridsearch(int L, const cdm::Geom& g, float* params, int ng
   return hipGetLastError();
 }
 
+// The search over basis signals: its kernel arguments and dynamic LDS at L
+// lanes per voxel (after the CFP table and the measurement cache: the table
+// values, the weight parameters' values, the voxels' rows).  A row stride of
+// L entries modulo 64 puts the groups of a wave on different banks.
+static constexpr size_t cdm_gs_table_max = 16 * 1024;
+
+static cdm_gs_plan op_gs_plan(int L, const cdm::Geom& g, const cdm::GridPlan& p, size_t* lds) {
+  cdm_gs_plan k;
+  std::memset(&k, 0, sizeof(k));
+  k.nshared = p.nshared;
+  k.nouter = p.nouter;
+  k.ninner = p.ninner;
+  unsigned grid = 0;
+  for (int i = 0; i < p.ngp; ++i) grid |= 1u << p.gparams[i];
+  k.grid = grid;
+  k.outer_vals = p.outer_vals;
+  k.inner_vals = p.inner_vals;
+  k.order = p.order;
+  const size_t table = (size_t)p.nshared * cdm_gs_ntab * sizeof(CDM_F64);
+  k.table_lds = (cdm_gs_table_dep & ~grid) == 0 && table > 0 && table <= cdm_gs_table_max ? 1 : 0;
+  k.table_fixed = (cdm_gs_table_dep & grid) == 0 ? 1 : 0;
+  k.frame_fixed = (cdm_gs_frame_dep & grid) == 0 ? 1 : 0;
+  size_t at = (op_lds(g) + 15) / 16 * 16;
+  k.off_common = (int)at;
+  at = (at + (size_t)g.nmeas * cdm_gs_nc * sizeof(cdm_tf) + 15) / 16 * 16;
+  k.off_table = (int)at;
+  if (k.table_lds) at += table;
+  k.off_inner = (int)at;
+  at = (at + (size_t)p.ninner * cdm_gs_nw * sizeof(float) + 15) / 16 * 16;
+  k.off_rows = (int)at;
+  const int n = cdm_gs_row * g.nmeas;
+  k.row_stride = n + ((cdm_gs_row * L - n % 64) % 64 + 64) % 64;
+  *lds = at + (size_t)(cdm_block / L) * k.row_stride * sizeof(cdm_tf);
+  return k;
+}
+
+static int op_grid_basis_lanes(int L, const cdm::Geom& g, const cdm::GridPlan& p) {
+  if constexpr (!cdm_gs_basis) return 0;
+  if ((size_t)p.ninner * cdm_gs_nw * sizeof(float) > cdm_gs_table_max) return 0;
+  for (; L <= 64; L *= 4) {
+    size_t lds = 0;
+    (void)op_gs_plan(L, g, p, &lds);
+    if (lds <= cdm_lds_max) return L;
+  }
+  return 0;
+}
+
+#ifdef CDM_GRID_LINEAR
+template <int L>
+static void op_gs_screen(const cdm_gs_args& a, const cdm_gs_plan& pl, size_t lds, const cdm_gs_work& wk, hipStream_t s) {
+  const dim3 grid = op_grid(a.g.nvox, L);
+  hipLaunchKernelGGL(cdm_gs_basis_kernel<L>, dim3(grid.x, (unsigned)wk.S), dim3(cdm_block), lds, s, a, pl, wk);
+}
+template <int L>
+static void op_gs_rescan(const cdm_gs_args& a, const cdm_gs_plan& pl, size_t lds, const cdm_gs_work& wk, int ncu,
+                         hipStream_t s) {
+  // at most every voxel's slices, else blocks that go through the list
+  const unsigned long long most = (unsigned long long)op_grid(a.g.nvox, L).x * (unsigned)wk.SB;
+  const unsigned long long cap = 8ull * (unsigned)(ncu > 0 ? ncu : 1);
+  hipLaunchKernelGGL(cdm_gs_basis_rescan_kernel<L>, dim3((unsigned)(most < cap ? most : cap)), dim3(cdm_block), lds, s,
+                     a, pl, wk);
+}
+#endif
+
+// L: a group size that op_grid_basis_lanes returned.
+static hipError_t op_gridsearch_basis(int L, const cdm::Geom& g, float* params, const cdm::GridPlan& p,
+                                      const cdm::Consts& c, int* kept, const cdm::GridWork& w, hipStream_t s) {
+#ifdef CDM_GRID_LINEAR
+  if (g.nvox <= 0) return hipSuccess;
+  if (p.ngp > cdm_np || g.cfp_ts > cdm_cfp_max || g.fixp_ts > cdm_fixp_max) return hipErrorInvalidValue;
+  cdm_gs_args a;
+  a.g = op_geom(g);
+  a.params = params;
+  a.ngp = p.ngp;
+  for (int i = 0; i < cdm_np; ++i) a.gparams[i] = i < p.ngp ? p.gparams[i] : -1;
+  a.ncombs = p.ncombs;
+  a.grid_f = p.grid_f;
+  a.grid_d = p.grid_d;
+  a.comb_id = p.comb_id;
+  a.c = op_consts(c);
+  a.kept_out = kept;
+  cdm_gs_work wk = {w.S, w.SB, w.part_c1, w.part_c2, w.part_i1, w.sumsq, w.count, w.list, w.thr, w.rescan_c, w.rescan_i};
+  size_t lds = 0;
+  const cdm_gs_plan pl = op_gs_plan(L, g, p, &lds);
+  hipLaunchKernelGGL(cdm_queue_reset_kernel, dim3(1), dim3(1), 0, s, w.count);
+  CDM_DISPATCH_L(L, op_gs_screen<LG>(a, pl, lds, wk, s));
+  if (wk.S > 1)
+    hipLaunchKernelGGL(cdm_gs_basis_merge_kernel, op_grid(g.nvox, cdm_gs_merge_lanes), dim3(cdm_block), 0, s, a, pl, wk);
+  // the FP64 scan runs on few voxels, at 16 lanes or more each
+  const int L2 = L < 16 ? 16 : L;
+  size_t lds2 = 0;
+  const cdm_gs_plan pl2 = op_gs_plan(L2, g, p, &lds2);
+  if (L2 == 16) op_gs_rescan<16>(a, pl2, lds2, wk, w.ncu, s);
+  else op_gs_rescan<64>(a, pl2, lds2, wk, w.ncu, s);
+  const unsigned pick = op_grid(g.nvox, cdm_gs_merge_lanes).x;
+  hipLaunchKernelGGL(cdm_gs_basis_pick_kernel, dim3(pick < 1024 ? pick : 1024), dim3(cdm_block), 0, s, a, wk);
+  return hipGetLastError();
+#else
+  return hipErrorInvalidValue;
+#endif
+}
+
 // Resident blocks per CU of the work-queue LM kernel <L, W> at `lds` bytes,
 // queried once per shape (host-side occupancy calculation).
 template <int L, int W>

@@ -17,16 +17,16 @@
 namespace cdm {
 
 __device__ __forceinline__ int lane_dpp_quad_xor1(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
+  return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);
 }
 __device__ __forceinline__ int lane_dpp_quad_xor2(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);
+  return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);
 }
 __device__ __forceinline__ int lane_dpp_half_mirror(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);
+  return __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true);
 }
 __device__ __forceinline__ int lane_dpp_mirror(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false);
+  return __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true);
 }
 __device__ __forceinline__ int lane_swz_xor16(int v) { return __builtin_amdgcn_ds_swizzle(v, 0x401F); }
 __device__ __forceinline__ int lane_xor32(int v) {

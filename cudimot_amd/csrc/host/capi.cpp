@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstring>
 #include <fstream>
+#include <map>
 #include <mutex>
 #include <sstream>
 #include <string>
@@ -63,6 +64,10 @@ struct cdm_model {
   float* d_grid_f = nullptr;
   double* d_grid_d = nullptr;
   int* d_comb_id = nullptr;
+  // the grid ordered for the search over basis signals (d_plan holds its
+  // tables; plan.order null: not a product, or the plug-in has no basis)
+  void* d_plan = nullptr;
+  cdm::GridPlan plan = {};
   // MCMC chain state
   void* d_state = nullptr;
   size_t state_bytes = 0;
@@ -282,6 +287,77 @@ void free_grid(cdm_model* m) {
   m->d_grid_f = nullptr;
   m->d_grid_d = nullptr;
   m->d_comb_id = nullptr;
+  if (m->d_plan) (void)hipFree(m->d_plan);
+  m->d_plan = nullptr;
+  m->plan = {};
+}
+
+// The grid's valid combinations (gf [n][ngp]) ordered by the plug-in's levels:
+// equal shared values together, within them equal values of every basis
+// parameter, each level in order of first appearance.  The search needs the
+// product structure a grid of per-parameter lists and per-parameter bounds
+// has; where it is not found the plan stays empty.
+int upload_plan(cdm_model* m, const std::vector<float>& gf, int n) {
+  const int ngp = (int)m->spec.grid_params.size();
+  if (!m->ops->grid_linear || n <= 0) return 0;
+  cdm::GridPlan p = {};
+  std::vector<int> cols[3];  // columns of the shared, the other basis and the weight parameters
+  for (int k = 0; k < ngp; ++k) {
+    const unsigned bit = 1u << m->spec.grid_params[k];
+    cols[(m->ops->grid_linear & bit) ? 2 : (m->ops->grid_shared & bit) ? 0 : 1].push_back(k);
+  }
+  // per level: each combination's index among the level's distinct tuples
+  std::vector<int> idx[3];
+  int count[3];
+  for (int l = 0; l < 3; ++l) {
+    std::map<std::vector<float>, int> seen;
+    idx[l].resize(n);
+    for (int c = 0; c < n; ++c) {
+      std::vector<float> key;
+      for (int k : cols[l]) key.push_back(gf[(size_t)c * ngp + k]);
+      idx[l][c] = seen.emplace(key, (int)seen.size()).first->second;
+    }
+    count[l] = (int)seen.size();
+  }
+  if ((long long)count[0] * count[1] * count[2] != n) return 0;
+  std::vector<int> order(n, -1);
+  for (int c = 0; c < n; ++c) {
+    const int at = (idx[0][c] * count[1] + idx[1][c]) * count[2] + idx[2][c];
+    if (order[at] >= 0) return 0;  // a repeated combination
+    order[at] = c;
+  }
+  const int np = m->ops->nparams;
+  std::vector<float> outer((size_t)count[0] * count[1] * np, 0.0f), inner((size_t)count[2] * np, 0.0f);
+  for (int o = 0; o < count[0] * count[1]; ++o)
+    for (int k = 0; k < ngp; ++k)
+      outer[(size_t)o * np + m->spec.grid_params[k]] = gf[(size_t)order[(size_t)o * count[2]] * ngp + k];
+  for (int j = 0; j < count[2]; ++j)
+    for (int k : cols[2]) inner[(size_t)j * np + m->spec.grid_params[k]] = gf[(size_t)order[j] * ngp + k];
+  const size_t nb = outer.size() * 4, ni = inner.size() * 4, no = order.size() * 4;
+  hipError_t e = hipMalloc(&m->d_plan, nb + ni + no);
+  if (e != hipSuccess) {
+    m->d_plan = nullptr;
+    return hip_fail(e, "grid");
+  }
+  char* d = (char*)m->d_plan;
+  if ((e = hipMemcpy(d, outer.data(), nb, hipMemcpyHostToDevice)) != hipSuccess ||
+      (e = hipMemcpy(d + nb, inner.data(), ni, hipMemcpyHostToDevice)) != hipSuccess ||
+      (e = hipMemcpy(d + nb + ni, order.data(), no, hipMemcpyHostToDevice)) != hipSuccess)
+    return hip_fail(e, "grid upload");
+  p.ngp = ngp;
+  p.ncombs = n;
+  p.gparams = m->spec.grid_params.data();
+  p.grid_f = m->d_grid_f;
+  p.grid_d = m->d_grid_d;
+  p.comb_id = m->d_comb_id;
+  p.nshared = count[0];
+  p.nouter = count[1];
+  p.ninner = count[2];
+  p.outer_vals = (const float*)d;
+  p.inner_vals = (const float*)(d + nb);
+  p.order = (const int*)(d + nb + ni);
+  m->plan = p;
+  return 0;
 }
 
 // Combinations whose grid values pass the float bounds test of
@@ -324,6 +400,8 @@ int upload_grid(cdm_model* m) {
       return hip_fail(e, "grid upload");
     if ((e = hipMemcpy(m->d_comb_id, id.data(), id.size() * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess)
       return hip_fail(e, "grid upload");
+    const int r = upload_plan(m, gf, m->ncombs_valid);
+    if (r) return r;
   }
   m->grid_dirty = false;
   return 0;
@@ -643,23 +721,59 @@ int cdm_model_set_mcmc_blocks(cdm_model* m, int jumps_per_launch, int use_graph)
   return 0;
 }
 
-// Slices of the combinations for a GridSearch whose voxel groups alone
-// leave the GPU mostly idle: enough (at most 16, at least 64 combinations
-// each) for about 8 blocks per CU; 1 for volumes that fill it.
-int gs_splits(int L, int nvox, int ncombs) {
+// Compute units of the current device (0 if unknown).
+static int device_cus() {
   int dev = 0, ncu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
     (void)hipGetLastError();
-    return 1;
+    return 0;
   }
+  return ncu;
+}
+
+// Slices of the combinations for a GridSearch whose voxel groups alone
+// leave the GPU mostly idle: enough (at most `most`, at least 64 combinations
+// each) for about 8 blocks per CU; 1 for volumes that fill it.
+int gs_splits(int L, int nvox, int ncombs, int most) {
+  const int ncu = device_cus();
+  if (ncu <= 0) return 1;
   const long long per_block = 256 / L;
   const long long blocks = ((long long)nvox + per_block - 1) / per_block;
   const long long target = 8LL * ncu;
   if (blocks >= target) return 1;
-  long long S = std::min<long long>(16, (target + blocks - 1) / blocks);
+  long long S = std::min<long long>(most, (target + blocks - 1) / blocks);
   S = std::min<long long>(S, std::max(1, ncombs / 64));
   return (int)std::max<long long>(1, S);
+}
+
+// The handle's GridSearch scratch, at least `bytes`, ordered after the
+// handle's last call (its previous user).
+static hipError_t gs_scratch(cdm_model* m, size_t bytes, hipStream_t s) {
+  hipError_t e = order_after_last(m, s);
+  if (e != hipSuccess || m->gs_split_bytes >= bytes) return e;
+  if (m->has_last && (e = hipStreamSynchronize(m->last_stream)) != hipSuccess) return e;
+  if (m->d_gs_split) (void)hipFree(m->d_gs_split);
+  m->d_gs_split = nullptr;
+  m->gs_split_bytes = 0;
+  if ((e = hipMalloc(&m->d_gs_split, bytes)) != hipSuccess) {
+    m->d_gs_split = nullptr;
+    return e;
+  }
+  m->gs_split_bytes = bytes;
+  return hipSuccess;
+}
+
+// Lanes per voxel of a search over basis signals: 4 (16 past 192
+// measurements, where a voxel's LDS rows get long), widened only when the
+// voxels and the slices of the shared combinations together leave lanes idle;
+// an explicit set_group stands.  0: the search does not apply.
+static int gs_basis_lanes(const cdm_model* m, const cdm::Geom& g) {
+  if (!m->plan.order) return 0;
+  int L = m->group[cdm::kGridSearch];
+  if (!L)
+    for (L = g.nmeas >= 192 ? 16 : 4; L < 64 && (long long)g.nvox * L * m->plan.nshared < kLaneSlots;) L *= 4;
+  return m->ops->grid_basis_lanes(L, g, m->plan);
 }
 
 int cdm_gridsearch(cdm_model* m, int nvox, int nmeas, const float* meas, float* params, const float* cfp,
@@ -672,27 +786,33 @@ int cdm_gridsearch(cdm_model* m, int nvox, int nmeas, const float* meas, float* 
   const cdm::Geom g = make_geom(m, nvox, nmeas, meas, cfp, fixp);
   const cdm::Consts c = make_consts(m);
   hipStream_t s = (hipStream_t)stream;
-  const int L = group_for(m, cdm::kGridSearch, nmeas, nvox);
-  const int S = gs_splits(L, nvox, m->ncombs_valid);
   hipError_t e = hipSuccess;
-  if (S > 1) {
-    // the lists belong to the handle: order after its last launch
-    const size_t bytes = cdm::gs_split_bytes(nvox, S);
-    if (m->gs_split_bytes < bytes) {
-      if ((e = order_after_last(m, s)) != hipSuccess) return hip_fail(e, "GridSearch stream order");
-      if (m->has_last && (e = hipStreamSynchronize(m->last_stream)) != hipSuccess)
-        return hip_fail(e, "GridSearch scratch");
-      if (m->d_gs_split) (void)hipFree(m->d_gs_split);
-      m->d_gs_split = nullptr;
-      m->gs_split_bytes = 0;
-      if ((e = hipMalloc(&m->d_gs_split, bytes)) != hipSuccess) {
-        m->d_gs_split = nullptr;
-        return hip_fail(e, "GridSearch scratch");
-      }
-      m->gs_split_bytes = bytes;
-    }
-    if ((e = order_after_last(m, s)) != hipSuccess) return hip_fail(e, "GridSearch stream order");
+  // The search over basis signals keeps its lists in the handle's scratch; a
+  // capturing caller gets the scan that needs none for a volume that fills
+  // the GPU.
+  hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cst) != hipSuccess) {
+    (void)hipGetLastError();
+    cst = hipStreamCaptureStatusActive;
   }
+  const int LB = cst == hipStreamCaptureStatusNone ? gs_basis_lanes(m, g) : 0;
+  if (LB) {
+    const int S = std::min(m->plan.nshared, gs_splits(LB, nvox, INT_MAX, m->plan.nshared));
+    const int SB = std::max(1, std::min(m->plan.nshared, (4 << 20) / nvox));
+    if ((e = gs_scratch(m, cdm::gs_work_bytes(nvox, S, SB), s)) != hipSuccess)
+      return hip_fail(e, "GridSearch scratch");
+    if ((e = debug_reset(m, 0, s)) != hipSuccess) return hip_fail(e, "GridSearch --debug records");
+    e = m->ops->gridsearch_basis(LB, g, params, m->plan, c, kept,
+                                 cdm::gs_work_of(m->d_gs_split, nvox, S, SB, device_cus()), s);
+    if (e != hipSuccess) return hip_fail(e, "GridSearch launch");
+    (void)note_last(m, s);
+    return 0;
+  }
+  const int L = group_for(m, cdm::kGridSearch, nmeas, nvox);
+  const int S = gs_splits(L, nvox, m->ncombs_valid, 16);
+  // the split search's lists belong to the handle too
+  if (S > 1 && (e = gs_scratch(m, cdm::gs_split_bytes(nvox, S), s)) != hipSuccess)
+    return hip_fail(e, "GridSearch scratch");
   if ((e = debug_reset(m, 0, s)) != hipSuccess) return hip_fail(e, "GridSearch --debug records");
   e = m->ops->gridsearch(L, g, params, (int)m->spec.grid_params.size(), m->spec.grid_params.data(), m->ncombs_valid,
                          m->d_grid_f, m->d_grid_d, m->d_comb_id, c, kept, S, S > 1 ? m->d_gs_split : nullptr, s);

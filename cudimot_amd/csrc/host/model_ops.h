@@ -53,6 +53,60 @@ inline size_t gs_split_bytes(int nvox, int S) {
   return n * (sizeof(double) + 4 * (sizeof(float) + sizeof(int)) + sizeof(int)) + (size_t)nvox * sizeof(int);
 }
 
+// A grid ordered for the search over basis signals: nshared combinations of
+// the plug-in's shared grid parameters, each with nouter of its other basis
+// parameters, each with ninner of its weight parameters (device pointers, as
+// the engine's cdm_gs_plan).
+struct GridPlan {
+  int ngp, ncombs;
+  const int* gparams;
+  const float* grid_f;
+  const double* grid_d;
+  const int* comb_id;
+  int nshared, nouter, ninner;
+  const float* outer_vals;  // [..][nparams]
+  const float* inner_vals;
+  const int* order;
+};
+
+// Scratch of that search: S screen slices, SB slices of the FP64 scan.
+struct GridWork {
+  int S, SB, ncu;
+  float *part_c1, *part_c2;
+  int* part_i1;
+  double* sumsq;
+  int* count;
+  int* list;
+  double* thr;
+  double* rescan_c;
+  int* rescan_i;
+};
+
+inline size_t gs_work_bytes(int nvox, int S, int SB) {
+  const size_t n = (size_t)nvox;
+  return n * SB * (sizeof(double) + sizeof(int)) + n * (2 * sizeof(double) + sizeof(int)) +
+         (S > 1 ? n * S * (2 * sizeof(float) + sizeof(int)) : 0) + 64;
+}
+
+// The parts of a gs_work_bytes buffer (doubles first).
+inline GridWork gs_work_of(void* buf, int nvox, int S, int SB, int ncu) {
+  const size_t n = (size_t)nvox;
+  GridWork w;
+  w.S = S;
+  w.SB = SB;
+  w.ncu = ncu;
+  w.rescan_c = (double*)buf;
+  w.thr = w.rescan_c + n * SB;
+  w.sumsq = w.thr + n;
+  w.count = (int*)(w.sumsq + n);
+  w.list = w.count + 16;
+  w.rescan_i = w.list + n;
+  w.part_i1 = w.rescan_i + n * SB;
+  w.part_c1 = (float*)(w.part_i1 + n * S);
+  w.part_c2 = w.part_c1 + n * S;
+  return w;
+}
+
 struct ModelOps {
   const char* name;
   int nparams;
@@ -81,6 +135,13 @@ struct ModelOps {
   // 1 when an MCMC launch of group size L keeps the per-measurement cache
   // rows in LDS (the state buffer then needs no rows after the chains)
   int (*mcmc_rows_lds)(int L, int W, const Geom& g);
+  // GridSearch over basis signals (plug-ins that declare CDM_GRID_LINEAR;
+  // grid_linear 0: not available): the parameters of its levels, the lanes a
+  // search of this shape runs at (0: its LDS does not fit), and the search
+  unsigned grid_linear, grid_shared;
+  int (*grid_basis_lanes)(int L, const Geom& g, const GridPlan& p);
+  hipError_t (*gridsearch_basis)(int L, const Geom& g, float* params, const GridPlan& p, const Consts& c, int* kept,
+                                 const GridWork& w, hipStream_t s);
 };
 
 // Voxel-group sizes compiled for every model and method.

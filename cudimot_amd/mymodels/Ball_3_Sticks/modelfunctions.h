@@ -30,6 +30,66 @@ MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
   return P[0] * s;
 }
 
+// GridSearch hooks: the signal is linear in the fractions and S0; the ball and the first two sticks
+// are shared by the combinations of the last stick's angles.
+#define CDM_GRID_LINEAR 0x125u        // S0, f1, f2, f3
+#define CDM_GRID_SHARED 0xDAu        // d, th1, ph1, th2, ph2
+#define CDM_GRID_SHARED_VALUES 3
+#define CDM_GRID_SHARED_BASIS 3
+#define CDM_GRID_OUTER_BASIS 1
+#define CDM_GRID_COMMON 4              // g, b
+#define CDM_GRID_FRAME 6
+#define CDM_GRID_FRAME_DEPENDS 0xD8u
+#define CDM_GRID_OUTER 3
+
+MACRO void b3s_axis(T th, T ph, T* n) {
+  T st, ct, sp, cp;
+  tsincos(th, &st, &ct);
+  tsincos(ph, &sp, &cp);
+  n[0] = st * cp;
+  n[1] = st * sp;
+  n[2] = ct;
+}
+
+MACRO T b3s_compartment(const T* CFP, T d, const T* n) {
+  const T g = CFP[0] * n[0] + CFP[1] * n[1] + CFP[2] * n[2];
+  return texp_fast(-(CFP[3] * d) * g * g);
+}
+
+MACRO void Grid_Frame(int npar, T* P, T* fr) {
+  b3s_axis(P[3], P[4], fr + 0);
+  b3s_axis(P[6], P[7], fr + 3);
+}
+
+MACRO void Grid_Shared(int npar, T* P, T* CFP, T* FixP, const double* tb, const T* fr, const double* mc, T* sh) {
+  sh[0] = texp_fast(-(CFP[3] * P[1]));
+  sh[1] = b3s_compartment(CFP, P[1], fr + 0);
+  sh[2] = b3s_compartment(CFP, P[1], fr + 3);
+}
+
+MACRO void Grid_Common(int npar, T* CFP, const double* mc, T* cm) {
+  for (int k = 0; k < 4; ++k) cm[k] = CFP[k];
+}
+
+MACRO void Grid_Shared_Basis(int npar, const T* sh, const T* cm, T* basis) {
+  basis[0] = sh[0];
+  basis[1] = sh[1];
+  basis[2] = sh[2];
+}
+
+MACRO void Grid_Outer(int npar, T* P, const double* tb, T* so) { b3s_axis(P[9], P[10], so); }
+
+MACRO void Grid_Outer_Basis(int npar, T* P, const T* cm, const T* so, const T* sh, T* basis) {
+  basis[0] = b3s_compartment(cm, P[1], so);
+}
+
+MACRO void Grid_Weights(int npar, T* P, T* FixP, T* w) {
+  w[0] = P[0] * ((T)1 - P[2] - P[5] - P[8]);
+  w[1] = P[0] * P[2];
+  w[2] = P[0] * P[5];
+  w[3] = P[0] * P[8];
+}
+
 MACRO bool ConstraintsMCMC(int npar, T* P) { return !(P[2] < P[5]) && !(P[5] < P[8]); }
 
 MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {

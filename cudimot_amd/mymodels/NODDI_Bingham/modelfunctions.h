@@ -27,6 +27,19 @@
 #define CDM_SIGNAL_PARTIALS 1               // signal and analytic entries together
 #define CDM_MEAS_CACHE 1                    // exp(-b Diso) per measurement
 #define CDM_LM_ROW_PASSES 2                 // 64-lane LM: the Jacobian rows in two passes
+// GridSearch: S = S0 (1-fiso) fan + S0 fiso iso; the intra-axonal signal and
+// the local gradient are shared by every fintra and fiso.
+#define CDM_GRID_LINEAR 0x01u          // fiso
+#define CDM_GRID_SHARED 0x7Cu          // kappa, beta, th, ph, psi
+#define CDM_GRID_SHARED_VALUES 3       // intra, cos^2 along the fibre, its complement's part along the azimuth
+#define CDM_GRID_SHARED_BASIS 1        // iso
+#define CDM_GRID_OUTER_BASIS 1         // fan
+#define CDM_GRID_COMMON 2              // b, iso
+#define CDM_GRID_TABLE 3               // normaliser and hindered moments of (kappa, beta)
+#define CDM_GRID_TABLE_DEPENDS 0x0Cu
+#define CDM_GRID_FRAME 9               // the fan's local frame
+#define CDM_GRID_FRAME_DEPENDS 0x70u
+#define CDM_GRID_OUTER 4               // fintra and the hindered diffusivities
 
 MACRO void Voxel_Cache(int npar, T* P, T* FixP, CDM_F64* vc) {
   bingham_fan f;
@@ -105,6 +118,58 @@ MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
   Voxel_Cache(npar, P, FixP, vc);
   Meas_Cache(CFP, mc);
   return Predicted_Signal_Cached(npar, P, CFP, FixP, vc, mc);
+}
+
+// GridSearch hooks: the same compartments from their shared parts.
+MACRO void Grid_Table(int npar, T* P, CDM_F64* tb) {
+  const CDM_F64 k = (CDM_F64)P[2], b = (CDM_F64)P[3];
+  CDM_F64 h[5];
+  for (int j = 0; j < 5; ++j) h[j] = bingham_fan_job(j, k, b);
+  tb[0] = log(4.0 * h[0]);
+  tb[1] = ((h[1] - h[2]) / (2.0 * bingham_fd_delta)) / h[0];
+  tb[2] = ((h[3] - h[4]) / (2.0 * bingham_fd_delta)) / h[0];
+}
+
+MACRO void Grid_Frame(int npar, T* P, T* fr) { bingham_fan_frame_of<T>(P[4], P[5], P[6], fr); }
+
+MACRO void Grid_Shared(int npar, T* P, T* CFP, T* FixP, const CDM_F64* tb, const T* fr, const CDM_F64* mc, T* sh) {
+  const T gx = CFP[0] * fr[0] + CFP[1] * fr[1] + CFP[2] * fr[2];
+  const T gy = CFP[0] * fr[3] + CFP[1] * fr[4] + CFP[2] * fr[5];
+  const T gn = CFP[0] * fr[6] + CFP[1] * fr[7] + CFP[2] * fr[8];
+  bingham_fan f;
+  f.lnc4 = tb[0];
+  sh[0] = bingham_fan_intra_local(P[2], P[3], gx, gy, gn, CFP[3], f);
+  const T c2 = gn * gn, s2 = (T)1 - c2, gxy = gx * gx + gy * gy;
+  const T caz2 = gxy > (T)0 ? tdiv_fast(gx * gx, gxy) : (T)1;
+  sh[1] = c2;
+  sh[2] = s2 * caz2;
+}
+
+MACRO void Grid_Common(int npar, T* CFP, const CDM_F64* mc, T* cm) {
+  cm[0] = CFP[3];
+  cm[1] = (T)mc[0];
+}
+
+MACRO void Grid_Shared_Basis(int npar, const T* sh, const T* cm, T* basis) { basis[0] = cm[1]; }
+
+MACRO void Grid_Outer(int npar, T* P, const CDM_F64* tb, T* so) {
+  const CDM_F64 dperp = CDM_NODDI_DPAR * (1.0 - (CDM_F64)P[1]), dd = CDM_NODDI_DPAR - dperp;
+  const CDM_F64 dpar = dperp + dd * tb[1], dperp1 = dperp + dd * tb[2];
+  so[0] = P[1];
+  so[1] = (T)dpar;
+  so[2] = (T)dperp1;
+  so[3] = (T)(CDM_NODDI_DPAR + 2 * dperp - dpar - dperp1);
+}
+
+MACRO void Grid_Outer_Basis(int npar, T* P, const T* cm, const T* so, const T* sh, T* basis) {
+  const T s2 = (T)1 - sh[1];
+  const T e = texp_fast(-cm[0] * (so[1] * sh[1] + (so[2] * (s2 - sh[2]) + so[3] * sh[2])));
+  basis[0] = ((T)1 - so[0]) * e + so[0] * sh[0];
+}
+
+MACRO void Grid_Weights(int npar, T* P, T* FixP, T* w) {
+  w[0] = FixP[0] * P[0];
+  w[1] = FixP[0] * ((T)1 - P[0]);
 }
 
 // kappa must exceed beta by 0.05 (NODDI_Bingham/modelfunctions.h:169-178).

@@ -18,6 +18,19 @@
 #define CDM_MEAS_CACHE 8               // L_0..L_6 (b Dpar), exp(-b Diso)
 #define CDM_NUMERICAL_MASK 0x1Cu       // kappa, th, ph
 #define CDM_SIGNAL_PARTIALS 1          // signal and analytic entries together
+// GridSearch: S = S0 (1-fiso) aniso + S0 fiso iso; the intra-axonal signal is
+// shared by every fintra and fiso.
+#define CDM_GRID_LINEAR 0x01u          // fiso
+#define CDM_GRID_SHARED 0x1Cu          // kappa, th, ph
+#define CDM_GRID_SHARED_VALUES 2       // intra, (g.n)^2
+#define CDM_GRID_SHARED_BASIS 1        // iso
+#define CDM_GRID_OUTER_BASIS 1         // aniso
+#define CDM_GRID_COMMON 2              // b, iso
+#define CDM_GRID_TABLE 8               // c_0..c_6, the hindered moment of kappa
+#define CDM_GRID_TABLE_DEPENDS 0x04u
+#define CDM_GRID_FRAME 3               // the fibre
+#define CDM_GRID_FRAME_DEPENDS 0x18u
+#define CDM_GRID_OUTER 3               // fintra and the hindered diffusivities
 
 MACRO void Voxel_Cache(int npar, T* P, T* FixP, CDM_F64* vc) {
   noddi_watson_hindered((CDM_F64)P[2], CDM_NODDI_DPAR * (1.0 - (CDM_F64)P[1]), vc[0], vc[1]);
@@ -63,6 +76,68 @@ MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
   Voxel_Cache(npar, P, FixP, vc);
   Meas_Cache(CFP, mc);
   return Predicted_Signal_Cached(npar, P, CFP, FixP, vc, mc);
+}
+
+// GridSearch hooks: the same compartments from their shared parts.
+MACRO void Grid_Table(int npar, T* P, CDM_F64* tb) {
+  noddi_watson_sh((CDM_F64)P[2], tb);
+  // dpar_eq of unit intra-axonal excess over zero perpendicular diffusivity:
+  // both hindered diffusivities are linear in dpar - dperp (Grid_Outer)
+  CDM_F64 dpar_eq, dperp_eq;
+  noddi_watson_hindered((CDM_F64)P[2], 0.0, dpar_eq, dperp_eq);
+  tb[7] = dpar_eq * (1.0 / CDM_NODDI_DPAR);
+}
+
+MACRO void Grid_Frame(int npar, T* P, T* fr) {
+  T st, ct, sp, cp;
+  tsincos(P[3], &st, &ct);
+  tsincos(P[4], &sp, &cp);
+  fr[0] = st * cp;
+  fr[1] = st * sp;
+  fr[2] = ct;
+}
+
+MACRO void Grid_Shared(int npar, T* P, T* CFP, T* FixP, const CDM_F64* tb, const T* fr, const CDM_F64* mc, T* sh) {
+  T gn = CFP[0] * fr[0] + CFP[1] * fr[1] + CFP[2] * fr[2];
+  sh[1] = gn * gn;
+  if (gn > (T)1) gn = (T)1;
+  if (gn < (T)-1) gn = (T)-1;
+  CDM_F64 p[7], s = 0.0;
+  noddi_even_legendre((CDM_F64)gn * (CDM_F64)gn, p);
+  const CDM_F64 norm[7] = {0.28209479177387814, 0.6307831305050401, 0.8462843753216345, 1.0171072362820548,
+                           1.1631066229203197,  1.2927207364566028, 1.4104739588693906};
+  for (int l = 0; l < 7; ++l) s += mc[l] * tb[l] * (norm[l] * p[l]);
+  if (s < 0) s = 1e-3;
+  sh[0] = (T)(0.5 * s);
+}
+
+MACRO void Grid_Common(int npar, T* CFP, const CDM_F64* mc, T* cm) {
+  cm[0] = CFP[3];
+  cm[1] = (T)mc[7];
+}
+
+MACRO void Grid_Shared_Basis(int npar, const T* sh, const T* cm, T* basis) { basis[0] = cm[1]; }
+
+MACRO void Grid_Outer(int npar, T* P, const CDM_F64* tb, T* so) {
+  const CDM_F64 dperp = CDM_NODDI_DPAR * (1.0 - (CDM_F64)P[1]), d = CDM_NODDI_DPAR - dperp;
+  const CDM_F64 dpar_eq = dperp + d * tb[7], dperp_eq = 0.5 * (CDM_NODDI_DPAR + dperp - d * tb[7]);
+  so[0] = P[1];
+  so[1] = (T)(dpar_eq - dperp_eq);
+  so[2] = (T)dperp_eq;
+}
+
+MACRO void Grid_Outer_Basis(int npar, T* P, const T* cm, const T* so, const T* sh, T* basis) {
+#ifdef CDM_WATSON_REFERENCE_FORMS
+  const T e = exp_gpu(-cm[0] * (so[1] * sh[1] + so[2]));
+#else
+  const T e = texp_fast(-cm[0] * (so[1] * sh[1] + so[2]));
+#endif
+  basis[0] = ((T)1 - so[0]) * e + so[0] * sh[0];
+}
+
+MACRO void Grid_Weights(int npar, T* P, T* FixP, T* w) {
+  w[0] = FixP[0] * P[0];
+  w[1] = FixP[0] * ((T)1 - P[0]);
 }
 
 MACRO bool ConstraintsMCMC(int npar, T* P) { return true; }

@@ -245,3 +245,18 @@ MACRO void noddi_even_sh(T x, T* sh) {
     if ((l & 1) == 0) sh[l / 2] = norm[l / 2] * p;
   }
 }
+
+// P_0, P_2, ..., P_12 at x^2 = x2, by the three-term recurrence of the even
+// polynomials (from x^2 P_n = A_n P_{n+2} + B_n P_n + C_n P_{n-2}).
+__device__ inline void noddi_even_legendre(CDM_F64 x2, CDM_F64* p) {
+  p[0] = 1.0;
+  p[1] = 1.5 * x2 - 0.5;
+#pragma unroll
+  for (int l = 1; l < 6; ++l) {
+    const double n = 2.0 * l;
+    const double A = (n + 1) * (n + 2) / ((2 * n + 1) * (2 * n + 3));
+    const double B = (n + 1) * (n + 1) / ((2 * n + 1) * (2 * n + 3)) + n * n / ((2 * n + 1) * (2 * n - 1));
+    const double C = n * (n - 1) / ((2 * n + 1) * (2 * n - 1));
+    p[l + 1] = (x2 * (1.0 / A) - B / A) * p[l] - (C / A) * p[l - 1];
+  }
+}

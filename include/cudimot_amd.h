@@ -16,7 +16,7 @@
  * `stream` is a hipStream_t (NULL: the null stream); calls are asynchronous
  * on it.  A model handle is not safe for concurrent use from several host
  * threads.  Its LM work-queue counter, MCMC chain state and GridSearch
- * scratch (small volumes) belong to the handle: such a call on another
+ * scratch belong to the handle: such a call on another
  * stream than the handle's previous one waits on the device for that call
  * to finish (outside stream capture; a capturing caller orders its streams
  * itself).  Use one handle per stream for concurrent fits.
@@ -115,9 +115,12 @@ int cdm_model_graph_stats(const cdm_model* m, long long* captures, long long* re
  * grid parameters of `params` to the combination of least squared error
  * (the FP64 argmin, earliest combination on ties).  kept (nullable,
  * device int[nvox]) receives the kept combination index, -1 if none.
- * Volumes too small to fill the GPU search slices of the combinations in
- * parallel, with the same result (scratch allocated on the handle at the
- * first such call of a larger size). */
+ * Plug-ins with GridSearch basis hooks (the shipped stick and NODDI models but
+ * NODDI_Bingham_2Fans) evaluate what combinations share once; other plug-ins,
+ * and calls under stream capture, scan every combination.  Volumes too small
+ * to fill the GPU search slices of the combinations in parallel.  The result is
+ * the same either way.  Scratch is allocated on the handle at the first call
+ * of a larger size (the scan of a volume that fills the GPU needs none). */
 int cdm_gridsearch(cdm_model* m, int nvox, int nmeas, const float* meas, float* params, const float* cfp,
                    const float* fixp, int* kept, void* stream);
 
