@@ -96,6 +96,7 @@ PLUGIN_MACROS = ["MODEL_H_INCLUDED", "NPARAMS", "NCFP", "NFIXP", "CDM_LM_JACOBIA
                  "CDM_MEAS_VOXEL_CACHE_FILL", "CDM_MEAS_VOXEL_CACHE_PARTIAL", "CDM_VOXEL_CACHE_PARTIAL", "CDM_SIGNAL_PARTIALS", "CDM_WATSON_REFERENCE_FORMS",
                  "CDM_LM_JACOBIAN_COLUMNS", "CDM_LM_ROW_PASSES", "CDM_GRID_LINEAR", "CDM_GRID_SHARED",
                  "CDM_GRID_SHARED_VALUES", "CDM_GRID_SHARED_BASIS", "CDM_GRID_OUTER_BASIS", "CDM_GRID_COMMON",
+                 "CDM_SIGNAL_FRAME", "CDM_SIGNAL_FRAME_DEPENDS",
                  "CDM_GRID_TABLE",
                  "CDM_GRID_TABLE_DEPENDS", "CDM_GRID_FRAME", "CDM_GRID_FRAME_DEPENDS", "CDM_GRID_OUTER"]
 

@@ -93,6 +93,17 @@ constexpr int cdm_ntri = cdm::tri_size(NPARAMS);
 //                              Predicted_Signal_Cached and fills the analytic
 //                              entries of Partial_Derivatives_Cached from one
 //                              evaluation of the shared parts
+//   CDM_SIGNAL_FRAME n         n values per parameter vector that depend on the
+//                              parameters in CDM_SIGNAL_FRAME_DEPENDS alone
+//                              (sines and cosines of the angles):
+//                              Signal_Frame(npar, P, fr, changed) recomputes the
+//                              entries that depend on parameter `changed`, and
+//                              Predicted_Signal_Framed(npar, P, CFP, FixP, vc, mc,
+//                              fr) (with CDM_MEAS_VOXEL_CACHE also
+//                              Predicted_Signal_MV_Framed and
+//                              Predicted_Signal_MV_Fill_Framed) give the values of
+//                              the plain forms from them.  MCMC keeps them per
+//                              voxel: a step recomputes only those it moves
 //   CDM_GRID_LINEAR b          GridSearch: the signal is a weighted sum of basis
 //                              signals, S = sum_k w_k B_k, and the parameters
 //                              in b enter the weights only
@@ -134,6 +145,13 @@ constexpr unsigned cdm_mvc_dep = CDM_MEAS_VOXEL_CACHE_DEPENDS;
 #else
 constexpr int cdm_mvc = 0;
 constexpr unsigned cdm_mvc_dep = 0;
+#endif
+#ifdef CDM_SIGNAL_FRAME
+constexpr int cdm_nframe = CDM_SIGNAL_FRAME;
+constexpr unsigned cdm_frame_dep = CDM_SIGNAL_FRAME_DEPENDS;
+#else
+constexpr int cdm_nframe = 0;
+constexpr unsigned cdm_frame_dep = 0;
 #endif
 // The column-wise LM Jacobian keeps the base point's per-measurement cache
 // values in LDS, so that a probe recomputes only the entries its parameter
@@ -2186,6 +2204,7 @@ struct cdm_vslot {
   CDM_F64 vc[cdm_vc_in_lds ? cdm_vc : 1];
   CDM_F64 jr[cdm_vc_in_lds && cdm_vc_jobs > 0 ? cdm_vc_jobs : 1];
   int nacc[cdm_np], nrej[cdm_np];
+  cdm_tf fr[cdm_nframe > 0 ? cdm_nframe : 1];  // the current state's Signal_Frame values
 };
 
 // Byte offset of the slots in the dynamic LDS (after the CFP table and the
@@ -2250,17 +2269,27 @@ __device__ __forceinline__ double cdm_logI0(double x) {
   return y;
 }
 
+// The signal with the frame's values, and the plain form without any.
+__device__ __forceinline__ cdm_tf cdm_signal_f(cdm_tf* p, cdm_tf* cfp, cdm_tf* fx, const CDM_F64* vc, const CDM_F64* mc,
+                                               const cdm_tf* fr) {
+#ifdef CDM_SIGNAL_FRAME
+  if (fr) return Predicted_Signal_Framed(cdm_np, p, cfp, fx, vc, mc, fr);
+#endif
+  return cdm_signal(p, cfp, fx, vc, mc);
+}
+
+// fr: the Signal_Frame values of p, or null (the plain signal).
 template <int L, bool RICIAN>
 __device__ __forceinline__ double cdm_neg_loglik(const cdm_geom& g, const float* s_cfp, const CDM_F64* s_mc,
                                                  const float* mv, const double* p, double tau, cdm_tf* fx,
-                                                 const CDM_F64* vc, int lane) {
+                                                 const CDM_F64* vc, int lane, const cdm_tf* fr = nullptr) {
   cdm_tf pf[cdm_np];
 #pragma unroll
   for (int i = 0; i < cdm_np; ++i) pf[i] = (cdm_tf)p[i];
   cdm_cfp_row<cdm_tf> row;
   double acc = 0.0;
   for (int m = lane; m < g.nmeas; m += L) {
-    const cdm_tf s = cdm_signal(pf, row.at(s_cfp, m, g.cfp_ts), fx, vc, cdm_mc_row(s_mc, m));
+    const cdm_tf s = cdm_signal_f(pf, row.at(s_cfp, m, g.cfp_ts), fx, vc, cdm_mc_row(s_mc, m), fr);
     if constexpr (RICIAN) {
       const double y = mv[m], sd = (double)s;
       acc += log(y) + (-0.5 * tau * (y * y + sd * sd) + cdm_logI0(tau * sd * y));
@@ -2280,8 +2309,9 @@ __device__ __forceinline__ double cdm_neg_loglik(const cdm_geom& g, const float*
 template <int L, bool RICIAN, int MODE>
 __device__ __forceinline__ double cdm_neg_loglik_mv(const cdm_geom& g, const float* s_cfp, const CDM_F64* s_mc,
                                                     const float* mv, const double* p, double tau, cdm_tf* fx,
-                                                    const CDM_F64* vc, cdm_tf* row, int lane,
+                                                    const CDM_F64* vc, cdm_tf* row, int lane, const cdm_tf* fr,
                                                     const cdm_tf* row_cur = nullptr, int changed = -1) {
+  (void)fr;
 #ifdef CDM_MEAS_VOXEL_CACHE
   cdm_tf pf[cdm_np];
 #pragma unroll
@@ -2299,6 +2329,8 @@ __device__ __forceinline__ double cdm_neg_loglik_mv(const cdm_geom& g, const flo
 #pragma unroll
       for (int k = 0; k < cdm_mvc; ++k) cur[k] = changed >= 0 ? row_cur[m * cdm_mvc + k] : (cdm_tf)0;
       s = Predicted_Signal_MV_Update(cdm_np, pf, cfpm, fx, vc, mcm, cur, mvc, changed);
+#elif defined(CDM_SIGNAL_FRAME)
+      s = Predicted_Signal_MV_Fill_Framed(cdm_np, pf, cfpm, fx, vc, mcm, mvc, fr);
 #elif defined(CDM_MEAS_VOXEL_CACHE_FILL)
       s = Predicted_Signal_MV_Fill(cdm_np, pf, cfpm, fx, vc, mcm, mvc);
 #else
@@ -2310,7 +2342,11 @@ __device__ __forceinline__ double cdm_neg_loglik_mv(const cdm_geom& g, const flo
     } else {
 #pragma unroll
       for (int k = 0; k < cdm_mvc; ++k) mvc[k] = row[m * cdm_mvc + k];
+#ifdef CDM_SIGNAL_FRAME
+      s = Predicted_Signal_MV_Framed(cdm_np, pf, cfpm, fx, vc, mcm, mvc, fr);
+#else
       s = Predicted_Signal_MV(cdm_np, pf, cfpm, fx, vc, mcm, mvc);
+#endif
     }
     if constexpr (RICIAN) {
       const double y = mv[m], sd = (double)s;
@@ -2324,9 +2360,14 @@ __device__ __forceinline__ double cdm_neg_loglik_mv(const cdm_geom& g, const flo
   if constexpr (RICIAN) return -g.nmeas * log(tau) - acc;
   else return (g.nmeas / 2.0) * log(acc / 2.0);
 #else
-  return cdm_neg_loglik<L, RICIAN>(g, s_cfp, s_mc, mv, p, tau, fx, vc, lane);
+  return cdm_neg_loglik<L, RICIAN>(g, s_cfp, s_mc, mv, p, tau, fx, vc, lane, fr);
 #endif
 }
+
+template <int M>
+struct cdm_mode {  // a mode passed as a type
+  static constexpr int value = M;
+};
 
 // Voxel cache of a double parameter vector, computed in the plug-in's precision.
 __device__ __forceinline__ void cdm_prepare_d(const double* p, cdm_tf* fx, CDM_F64* vc) {
@@ -2487,22 +2528,53 @@ __device__ __forceinline__ void cdm_mcmc_body(const cdm_mcmc_args& a, int block)
   // state's; in the block's LDS when they fit there, else in global memory.
   // Each lane reads only the entries it wrote itself, so neither needs a
   // barrier; row 0 is filled at the start of every launch.
-  cdm_tf* mvc_rows = nullptr;
+  // Two pointers, of which one is used: a pointer that may be either makes
+  // every access a flat one.
+  cdm_tf *rows_lds = nullptr, *rows_mem = nullptr;
   size_t rs = 0;
   if constexpr (cdm_mvc > 0) {
-    if (a.rows_lds) {
-      rs = (size_t)a.row_stride;
-      mvc_rows = reinterpret_cast<cdm_tf*>(reinterpret_cast<char*>(s_cfp) +
-                                           cdm_mcmc_rows_offset(a.g.nmeas, a.g.cfp_ts, L)) +
-                 (size_t)(threadIdx.x / L) * 2 * rs;
-    } else {
-      rs = (size_t)a.g.nmeas * cdm_mvc;
-      mvc_rows = a.mvc + (size_t)v * 2 * rs;
-    }
+    rs = a.rows_lds ? (size_t)a.row_stride : (size_t)a.g.nmeas * cdm_mvc;
+    rows_lds = reinterpret_cast<cdm_tf*>(reinterpret_cast<char*>(s_cfp) +
+                                         cdm_mcmc_rows_offset(a.g.nmeas, a.g.cfp_ts, L)) +
+               (size_t)(threadIdx.x / L) * 2 * rs;
+    rows_mem = a.mvc + (size_t)v * 2 * rs;
   }
   int cur = 0;
-  if constexpr (cdm_mvc > 0)
-    (void)cdm_neg_loglik_mv<L, RICIAN, 2>(a.g, s_cfp, s_mc, mv, p, tau, fx, vc_cur, mvc_rows, lane);
+  // the frame values of the current state, in the voxel's slot
+#ifdef CDM_SIGNAL_FRAME
+  {
+    cdm_tf pf[cdm_np], fr0[cdm_nframe];
+#pragma unroll
+    for (int k = 0; k < cdm_np; ++k) pf[k] = (cdm_tf)p[k];
+#pragma unroll
+    for (int k = 0; k < cdm_nframe; ++k) fr0[k] = (cdm_tf)0;
+#pragma unroll 1
+    for (int k = 0; k < cdm_np; ++k)
+      if ((cdm_frame_dep >> k) & 1u) Signal_Frame(cdm_np, pf, fr0, k);
+#pragma unroll
+    for (int k = 0; k < cdm_nframe; ++k) vs->fr[k] = fr0[k];
+  }
+#endif
+  cdm_tf fr_buf[cdm_nframe > 0 ? cdm_nframe : 1];
+  const cdm_tf* fr = cdm_nframe > 0 ? fr_buf : nullptr;
+  auto load_frame = [&]() {
+#pragma unroll
+    for (int k = 0; k < cdm_nframe; ++k) fr_buf[k] = vs->fr[k];
+  };
+  // likelihood through the cache rows: MODE 1 reads row `from`, MODE 2 fills it
+  // after a step in `changed` from row `old`
+  auto like_rows = [&](auto mode, const CDM_F64* vcx, int row, int old, int changed) {
+    constexpr int MODE = decltype(mode)::value;
+    if (a.rows_lds)
+      return cdm_neg_loglik_mv<L, RICIAN, MODE>(a.g, s_cfp, s_mc, mv, p, tau, fx, vcx, rows_lds + row * rs, lane, fr,
+                                                rows_lds + old * rs, changed);
+    return cdm_neg_loglik_mv<L, RICIAN, MODE>(a.g, s_cfp, s_mc, mv, p, tau, fx, vcx, rows_mem + row * rs, lane, fr,
+                                              rows_mem + old * rs, changed);
+  };
+  if constexpr (cdm_mvc > 0) {
+    load_frame();
+    (void)like_rows(cdm_mode<2>(), vc_cur, 0, 0, -1);
+  }
   const int end = a.begin + a.count;
   for (int it = a.begin; it < end; ++it) {
     const uint32_t jump = a.jump_offset + (uint32_t)it;
@@ -2547,10 +2619,11 @@ __device__ __forceinline__ void cdm_mcmc_body(const cdm_mcmc_args& a, int block)
         double tp = 0.0;
 #pragma unroll
         for (int i = 0; i < cdm_np; ++i) tp += prior[i];
-        const double e_new =
-            tp + (cdm_mvc > 0 ? cdm_neg_loglik_mv<L, true, 1>(a.g, s_cfp, s_mc, mv, p, tau, fx, vc_cur,
-                                                              mvc_rows + cur * rs, lane)
-                              : cdm_neg_loglik<L, true>(a.g, s_cfp, s_mc, mv, p, tau, fx, vc_cur, lane));
+        load_frame();
+        double like;
+        if constexpr (cdm_mvc > 0) like = like_rows(cdm_mode<1>(), vc_cur, cur, cur, -1);
+        else like = cdm_neg_loglik<L, true>(a.g, s_cfp, s_mc, mv, p, tau, fx, vc_cur, lane, fr);
+        const double e_new = tp + like;
         if (exp(energy - e_new) > d.uniform) {
           ++tau_acc;
           energy = e_new;
@@ -2613,14 +2686,20 @@ __device__ __forceinline__ void cdm_mcmc_body(const cdm_mcmc_args& a, int block)
         CDM_F64 vcu[cdm_vc];
 #pragma unroll
         for (int k = 0; k < cdm_vc; ++k) vcu[k] = dep ? vc_new[k] : vc_cur[k];
+        load_frame();
+#ifdef CDM_SIGNAL_FRAME
+        if ((cdm_frame_dep >> i) & 1u) {
+          cdm_tf pf[cdm_np];
+#pragma unroll
+          for (int k = 0; k < cdm_np; ++k) pf[k] = (cdm_tf)p[k];
+          Signal_Frame(cdm_np, pf, fr_buf, i);
+        }
+#endif
         double like;
         if constexpr (cdm_mvc > 0) {
-          like = mdep ? cdm_neg_loglik_mv<L, RICIAN, 2>(a.g, s_cfp, s_mc, mv, p, tau, fx, vcu,
-                                                        mvc_rows + (1 - cur) * rs, lane, mvc_rows + cur * rs, i)
-                      : cdm_neg_loglik_mv<L, RICIAN, 1>(a.g, s_cfp, s_mc, mv, p, tau, fx, vcu, mvc_rows + cur * rs,
-                                                        lane);
+          like = mdep ? like_rows(cdm_mode<2>(), vcu, 1 - cur, cur, i) : like_rows(cdm_mode<1>(), vcu, cur, cur, -1);
         } else {
-          like = cdm_neg_loglik<L, RICIAN>(a.g, s_cfp, s_mc, mv, p, tau, fx, vcu, lane);
+          like = cdm_neg_loglik<L, RICIAN>(a.g, s_cfp, s_mc, mv, p, tau, fx, vcu, lane, fr);
         }
         const double old_prior = prior[i];
         prior[i] = cdm_prior(a.c, i, p, a.g.nmeas, s_cfp, fx);
@@ -2638,6 +2717,10 @@ __device__ __forceinline__ void cdm_mcmc_body(const cdm_mcmc_args& a, int block)
             for (int j = 0; j < cdm_vc_jobs; ++j) jr_cur[j] = (dep && jdep) ? jr_new[j] : jr_cur[j];
           }
           if (mdep) cur = 1 - cur;
+          if ((cdm_frame_dep >> i) & 1u) {
+#pragma unroll
+            for (int k = 0; k < cdm_nframe; ++k) vs->fr[k] = fr_buf[k];
+          }
         } else {
           ++nrej[i];
           p[i] = old;

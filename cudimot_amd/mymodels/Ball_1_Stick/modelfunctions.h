@@ -27,6 +27,34 @@ MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
   return P[0] * (((T)1 - P[2]) * ball + P[2] * stick);
 }
 
+// MCMC hooks: the signal from the sines and cosines of the sticks' angles.
+#define CDM_SIGNAL_FRAME 4
+#define CDM_SIGNAL_FRAME_DEPENDS 0x18u
+
+MACRO void Signal_Frame(int npar, T* P, T* fr, int changed) {
+  const int angle[2] = {3, 4};
+  T s, c;
+  tsincos(changed == 3 ? P[3] : P[4], &s, &c);
+  for (int k = 0; k < 2; ++k) {
+    if (changed != angle[k]) continue;
+    fr[2 * k] = s;
+    fr[2 * k + 1] = c;
+  }
+}
+
+MACRO T b1s_along(const T* CFP, const T* tr) {
+  const T gxy = CFP[0] * tr[3] + CFP[1] * tr[2];
+  return tr[0] * gxy + CFP[2] * tr[1];
+}
+
+MACRO T Predicted_Signal_Framed(int npar, T* P, T* CFP, T* FixP, const double* vc, const double* mc, const T* fr) {
+  const T gn = b1s_along(CFP, fr);
+  const T bd = CFP[3] * P[1];
+  const T ball = texp_fast(-bd);
+  const T stick = texp_fast(-bd * gn * gn);
+  return P[0] * (((T)1 - P[2]) * ball + P[2] * stick);
+}
+
 // GridSearch hooks: the signal is linear in the fractions and S0; the ball
 // are shared by the combinations of the last stick's angles.
 #define CDM_GRID_LINEAR 0x05u        // S0, f

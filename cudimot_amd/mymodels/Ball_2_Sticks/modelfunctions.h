@@ -34,6 +34,35 @@ MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
   return P[0] * (((T)1 - P[2] - P[5]) * ball + P[2] * s1 + P[5] * s2);
 }
 
+// MCMC hooks: the signal from the sines and cosines of the sticks' angles.
+#define CDM_SIGNAL_FRAME 8
+#define CDM_SIGNAL_FRAME_DEPENDS 0xD8u
+
+MACRO void Signal_Frame(int npar, T* P, T* fr, int changed) {
+  const int angle[4] = {3, 4, 6, 7};
+  T s, c;
+  tsincos(changed == 3 ? P[3] : changed == 4 ? P[4] : changed == 6 ? P[6] : P[7], &s, &c);
+  for (int k = 0; k < 4; ++k) {
+    if (changed != angle[k]) continue;
+    fr[2 * k] = s;
+    fr[2 * k + 1] = c;
+  }
+}
+
+MACRO T b2s_along(const T* CFP, const T* tr) {
+  const T gxy = CFP[0] * tr[3] + CFP[1] * tr[2];
+  return tr[0] * gxy + CFP[2] * tr[1];
+}
+
+MACRO T Predicted_Signal_Framed(int npar, T* P, T* CFP, T* FixP, const double* vc, const double* mc, const T* fr) {
+  const T g1 = b2s_along(CFP, fr), g2 = b2s_along(CFP, fr + 4);
+  const T bd = CFP[3] * P[1];
+  const T ball = texp_fast(-bd);
+  const T s1 = texp_fast(-bd * g1 * g1);
+  const T s2 = texp_fast(-bd * g2 * g2);
+  return P[0] * (((T)1 - P[2] - P[5]) * ball + P[2] * s1 + P[5] * s2);
+}
+
 // GridSearch hooks: the signal is linear in the fractions and S0; the ball and the first stick
 // are shared by the combinations of the last stick's angles.
 #define CDM_GRID_LINEAR 0x25u        // S0, f1, f2

@@ -30,6 +30,37 @@ MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
   return P[0] * s;
 }
 
+// MCMC hooks: the signal from the sines and cosines of the sticks' angles.
+#define CDM_SIGNAL_FRAME 12
+#define CDM_SIGNAL_FRAME_DEPENDS 0x6D8u
+
+MACRO void Signal_Frame(int npar, T* P, T* fr, int changed) {
+  const int angle[6] = {3, 4, 6, 7, 9, 10};
+  T s, c;
+  tsincos(changed == 3 ? P[3] : changed == 4 ? P[4] : changed == 6 ? P[6] : changed == 7 ? P[7] : changed == 9 ? P[9] : P[10], &s, &c);
+  for (int k = 0; k < 6; ++k) {
+    if (changed != angle[k]) continue;
+    fr[2 * k] = s;
+    fr[2 * k + 1] = c;
+  }
+}
+
+MACRO T b3s_along(const T* CFP, const T* tr) {
+  const T gxy = CFP[0] * tr[3] + CFP[1] * tr[2];
+  return tr[0] * gxy + CFP[2] * tr[1];
+}
+
+MACRO T Predicted_Signal_Framed(int npar, T* P, T* CFP, T* FixP, const double* vc, const double* mc, const T* fr) {
+  const T bd = CFP[3] * P[1];
+  T s = ((T)1 - P[2] - P[5] - P[8]) * texp_fast(-bd);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const T g = b3s_along(CFP, fr + 4 * k);
+    s += P[2 + 3 * k] * texp_fast(-bd * g * g);
+  }
+  return P[0] * s;
+}
+
 // GridSearch hooks: the signal is linear in the fractions and S0; the ball and the first two sticks
 // are shared by the combinations of the last stick's angles.
 #define CDM_GRID_LINEAR 0x125u        // S0, f1, f2, f3

@@ -202,17 +202,23 @@ __device__ inline void bingham_fan_setup(CDM_F64 fintra, CDM_F64 kappa, CDM_F64 
 // Gradient in the fan's local frame for measurement CFP (g, b): components
 // along the fibre n(th, ph), the fanning direction (from psi) and their cross
 // product (NODDI_Bingham/modelfunctions.h:116-138).
-MACRO void bingham_fan_local(T th, T ph, T psi, T* CFP, T& gx, T& gy, T& gn) {
-  T st, ct, sp, cp, ss, cs;
-  tsincos(th, &st, &ct);
-  tsincos(ph, &sp, &cp);
-  tsincos(psi, &ss, &cs);
+// tr: sine and cosine of th, of ph and of psi.
+MACRO void bingham_trig_local(const T* tr, T* CFP, T& gx, T& gy, T& gn) {
+  const T st = tr[0], ct = tr[1], sp = tr[2], cp = tr[3], ss = tr[4], cs = tr[5];
   const T n0 = st * cp, n1 = st * sp, n2 = ct;
   const T f0 = -cs * sp - ct * cp * ss, f1 = cp * cs - ct * sp * ss, f2 = st * ss;
   const T gx_local0 = f1 * n2 - f2 * n1, gx_local1 = f2 * n0 - f0 * n2, gx_local2 = f0 * n1 - f1 * n0;
   gn = CFP[0] * n0 + CFP[1] * n1 + CFP[2] * n2;       // along the fibre
   gy = CFP[0] * f0 + CFP[1] * f1 + CFP[2] * f2;       // along the fanning direction
   gx = CFP[0] * gx_local0 + CFP[1] * gx_local1 + CFP[2] * gx_local2;
+}
+
+MACRO void bingham_fan_local(T th, T ph, T psi, T* CFP, T& gx, T& gy, T& gn) {
+  T tr[6];
+  tsincos(th, &tr[0], &tr[1]);
+  tsincos(ph, &tr[2], &tr[3]);
+  tsincos(psi, &tr[4], &tr[5]);
+  bingham_trig_local(tr, CFP, gx, gy, gn);
 }
 
 // The same frame once per parameter vector, in the precision F: fr[0..2] =

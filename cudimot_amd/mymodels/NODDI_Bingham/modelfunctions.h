@@ -26,6 +26,8 @@
 #define CDM_MEAS_VOXEL_CACHE_FILL 1         // cache row and signal together
 #define CDM_SIGNAL_PARTIALS 1               // signal and analytic entries together
 #define CDM_MEAS_CACHE 1                    // exp(-b Diso) per measurement
+#define CDM_SIGNAL_FRAME 6                  // sine and cosine of th, ph, psi
+#define CDM_SIGNAL_FRAME_DEPENDS 0x70u
 #define CDM_LM_ROW_PASSES 2                 // 64-lane LM: the Jacobian rows in two passes
 // GridSearch: S = S0 (1-fiso) fan + S0 fiso iso; the intra-axonal signal and
 // the local gradient are shared by every fintra and fiso.
@@ -102,6 +104,53 @@ MACRO T Predicted_Signal_MV(int npar, T* P, T* CFP, T* FixP, const CDM_F64* vc, 
   const T fan = ((T)1 - P[1]) * e + P[1] * mvc[0];
   const T iso = (T)mc[0];
   return FixP[0] * (((T)1 - P[0]) * fan + P[0] * iso);
+}
+
+// The same from the sines and cosines of the angles (the frame).
+MACRO void Signal_Frame(int npar, T* P, T* fr, int changed) {
+  T s, c;
+  tsincos(changed == 4 ? P[4] : changed == 5 ? P[5] : P[6], &s, &c);
+  for (int k = 0; k < 3; ++k) {
+    if (changed != 4 + k) continue;
+    fr[2 * k] = s;
+    fr[2 * k + 1] = c;
+  }
+}
+
+MACRO T Predicted_Signal_MV_Framed(int npar, T* P, T* CFP, T* FixP, const CDM_F64* vc, const CDM_F64* mc, const T* mvc,
+                                   const T* fr) {
+  bingham_fan f;
+  f.lnc4 = vc[0];
+  f.dpar = vc[1];
+  f.dperp1 = vc[2];
+  f.dperp2 = vc[3];
+  T gx, gy, gn;
+  bingham_trig_local(fr, CFP, gx, gy, gn);
+  const T e = bingham_fan_extra_local(gx, gy, gn, CFP[3], f);
+  const T fan = ((T)1 - P[1]) * e + P[1] * mvc[0];
+  const T iso = (T)mc[0];
+  return FixP[0] * (((T)1 - P[0]) * fan + P[0] * iso);
+}
+
+MACRO T Predicted_Signal_MV_Fill_Framed(int npar, T* P, T* CFP, T* FixP, const CDM_F64* vc, const CDM_F64* mc, T* mvc,
+                                        const T* fr) {
+  bingham_fan f;
+  f.lnc4 = vc[0];
+  f.dpar = vc[1];
+  f.dperp1 = vc[2];
+  f.dperp2 = vc[3];
+  T gx, gy, gn;
+  bingham_trig_local(fr, CFP, gx, gy, gn);
+  const T e = bingham_fan_extra_local(gx, gy, gn, CFP[3], f);
+  mvc[0] = bingham_fan_intra_local(P[2], P[3], gx, gy, gn, CFP[3], f);
+  const T fan = ((T)1 - P[1]) * e + P[1] * mvc[0];
+  const T iso = (T)mc[0];
+  return FixP[0] * (((T)1 - P[0]) * fan + P[0] * iso);
+}
+
+MACRO T Predicted_Signal_Framed(int npar, T* P, T* CFP, T* FixP, const CDM_F64* vc, const CDM_F64* mc, const T* fr) {
+  T mvc[1];
+  return Predicted_Signal_MV_Fill_Framed(npar, P, CFP, FixP, vc, mc, mvc, fr);
 }
 
 // Meas_Voxel_Cache and Predicted_Signal_MV from one local gradient.

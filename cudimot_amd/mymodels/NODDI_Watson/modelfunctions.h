@@ -18,6 +18,8 @@
 #define CDM_MEAS_CACHE 8               // L_0..L_6 (b Dpar), exp(-b Diso)
 #define CDM_NUMERICAL_MASK 0x1Cu       // kappa, th, ph
 #define CDM_SIGNAL_PARTIALS 1          // signal and analytic entries together
+#define CDM_SIGNAL_FRAME 4             // sine and cosine of th, ph
+#define CDM_SIGNAL_FRAME_DEPENDS 0x18u
 // GridSearch: S = S0 (1-fiso) aniso + S0 fiso iso; the intra-axonal signal is
 // shared by every fintra and fiso.
 #define CDM_GRID_LINEAR 0x01u          // fiso
@@ -42,10 +44,9 @@ MACRO void Meas_Cache(T* CFP, CDM_F64* mc) {
   mc[7] = exp(-(CDM_F64)CFP[3] * CDM_NODDI_DISO);
 }
 
-MACRO void watson_parts(T* P, T* CFP, const CDM_F64* vc, const CDM_F64* mc, T& extra, T& intra) {
-  T st, ct, sp, cp;
-  tsincos(P[3], &st, &ct);
-  tsincos(P[4], &sp, &cp);
+// tr: sine and cosine of th and of ph.
+MACRO void watson_parts_of(const T* tr, T* P, T* CFP, const CDM_F64* vc, const CDM_F64* mc, T& extra, T& intra) {
+  const T st = tr[0], ct = tr[1], sp = tr[2], cp = tr[3];
   T gn = CFP[0] * st * cp + CFP[1] * st * sp + CFP[2] * ct;
 #ifdef CDM_WATSON_REFERENCE_FORMS
   extra = exp_gpu(-CFP[3] * ((T)(vc[0] - vc[1]) * gn * gn + (T)vc[1]));
@@ -62,6 +63,30 @@ MACRO void watson_parts(T* P, T* CFP, const CDM_F64* vc, const CDM_F64* mc, T& e
   for (int l = 0; l < 7; ++l) s += mc[l] * vc[2 + l] * (CDM_F64)sh[l];
   if (s < 0) s = 1e-3;
   intra = (T)(0.5 * s);
+}
+
+MACRO void watson_parts(T* P, T* CFP, const CDM_F64* vc, const CDM_F64* mc, T& extra, T& intra) {
+  T tr[4];
+  tsincos(P[3], &tr[0], &tr[1]);
+  tsincos(P[4], &tr[2], &tr[3]);
+  watson_parts_of(tr, P, CFP, vc, mc, extra, intra);
+}
+
+MACRO void Signal_Frame(int npar, T* P, T* fr, int changed) {
+  T s, c;
+  tsincos(changed == 3 ? P[3] : P[4], &s, &c);
+  for (int k = 0; k < 2; ++k) {
+    if (changed != 3 + k) continue;
+    fr[2 * k] = s;
+    fr[2 * k + 1] = c;
+  }
+}
+
+MACRO T Predicted_Signal_Framed(int npar, T* P, T* CFP, T* FixP, const CDM_F64* vc, const CDM_F64* mc, const T* fr) {
+  T extra, intra;
+  watson_parts_of(fr, P, CFP, vc, mc, extra, intra);
+  const T aniso = ((T)1 - P[1]) * extra + P[1] * intra;
+  return FixP[0] * (((T)1 - P[0]) * aniso + P[0] * (T)mc[7]);
 }
 
 MACRO T Predicted_Signal_Cached(int npar, T* P, T* CFP, T* FixP, const CDM_F64* vc, const CDM_F64* mc) {
