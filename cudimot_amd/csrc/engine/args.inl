@@ -108,6 +108,9 @@ static cdm_mcmc_args op_mcmc_args(const cdm::Geom& g, int L, int W, const cdm::M
   a.begin = m.begin;
   a.count = m.count;
   a.phase_len = m.phase_len;
+  a.queue = nullptr;
+  a.ntiles = (int)op_grid(g.nvox, L).x;
+  a.chunk_len = m.count;
   a.jump_offset = m.jump_offset;
   a.seed = m.seed;
   a.voxel_offset = m.voxel_offset;

@@ -153,7 +153,7 @@ static hipError_t op_gridsearch_basis(int L, const cdm::Geom& g, float* params, 
   cdm_gs_work wk = {w.S, w.SB, w.part_c1, w.part_c2, w.part_i1, w.sumsq, w.count, w.list, w.thr, w.rescan_c, w.rescan_i};
   size_t lds = 0;
   const cdm_gs_plan pl = op_gs_plan(L, g, p, &lds);
-  hipLaunchKernelGGL(cdm_queue_reset_kernel, dim3(1), dim3(1), 0, s, w.count);
+  hipLaunchKernelGGL(cdm_queue_reset_kernel, dim3(1), dim3(cdm_block), 0, s, w.count, 1);
   CDM_DISPATCH_L(L, op_gs_screen<LG>(a, pl, lds, wk, s));
   if (wk.S > 1)
     hipLaunchKernelGGL(cdm_gs_basis_merge_kernel, op_grid(g.nvox, cdm_gs_merge_lanes), dim3(cdm_block), 0, s, a, pl, wk);
@@ -212,9 +212,40 @@ static hipError_t op_levmar(int L, int W, const cdm::Geom& g, float* params, int
     return hipGetLastError();
   }
   a.queue = queue;
-  hipLaunchKernelGGL(cdm_queue_reset_kernel, dim3(1), dim3(1), 0, s, queue);
+  hipLaunchKernelGGL(cdm_queue_reset_kernel, dim3(1), dim3(cdm_block), 0, s, queue, 1);
   const size_t lds = op_lds_lm(g, L);
   CDM_DISPATCH_L(L, CDM_DISPATCH_W(W, (op_levmar_queue_launch<LG, WG>(a, marquardt, g.nvox, lds, ncu, s))));
+  return hipGetLastError();
+}
+
+// One MCMC launch: in time slices (cdm_mcmc_kernel) when the tiles outnumber the
+// resident blocks R without filling sixteen rounds of them, so that the last
+// round is at most a sixteenth of the launch; at least 16 jumps a slice, since
+// each slice rebuilds the voxel caches and cache rows (about 0.3 jumps).
+constexpr int cdm_mcmc_rounds = 16, cdm_mcmc_least_jumps = 16;
+
+template <int L, bool RICIAN, int W>
+static hipError_t op_mcmc_launch(cdm_mcmc_args a, size_t lds, int* queue, int ncu, hipStream_t s) {
+  dim3 grid((unsigned)a.ntiles);
+  if (queue && ncu > 0 && a.ntiles > ncu) {
+    int per_cu = 0;
+    const hipError_t e =
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (cdm_mcmc_kernel<L, RICIAN, W>), cdm_block, lds);
+    if (e != hipSuccess) return e;
+    const long long resident = (long long)per_cu * ncu;
+    const long long want = (cdm_mcmc_rounds * resident + a.ntiles - 1) / a.ntiles;
+    const int n = (int)std::min<long long>(want, a.count / cdm_mcmc_least_jumps);
+    if (resident > 0 && a.ntiles > resident && n > 1) {
+      a.queue = queue;
+      a.chunk_len = (a.count + n - 1) / n;
+      const unsigned slices = (unsigned)((a.count + a.chunk_len - 1) / a.chunk_len);
+      const int ints = 16 + a.ntiles;
+      hipLaunchKernelGGL(cdm_queue_reset_kernel, dim3((unsigned)((ints + cdm_block - 1) / cdm_block)),
+                         dim3(cdm_block), 0, s, queue, ints);
+      grid = dim3((unsigned)a.ntiles * slices);
+    }
+  }
+  hipLaunchKernelGGL((cdm_mcmc_kernel<L, RICIAN, W>), grid, dim3(cdm_block), lds, s, a);
   return hipGetLastError();
 }
 
@@ -225,14 +256,13 @@ static hipError_t op_mcmc(int L, int W, int rician, const cdm::Geom& g, const cd
   // the Rician likelihood is compiled at the default register budget only
   const int We = rician ? 1 : W;
   const cdm_mcmc_args a = op_mcmc_args(g, L, We, m, c);
+  const size_t lds = op_lds_mcmc(g, L, We);
   if (rician) {
-    CDM_DISPATCH_L(L, hipLaunchKernelGGL((cdm_mcmc_kernel<LG, true, 1>), op_grid(g.nvox, LG), dim3(cdm_block),
-                                         op_lds_mcmc(g, LG, We), s, a));
+    CDM_DISPATCH_L(L, return (op_mcmc_launch<LG, true, 1>(a, lds, m.queue, m.ncu, s)));
   } else {
-    CDM_DISPATCH_L(L, CDM_DISPATCH_W(W, hipLaunchKernelGGL((cdm_mcmc_kernel<LG, false, WG>), op_grid(g.nvox, LG),
-                                                           dim3(cdm_block), op_lds_mcmc(g, LG, We), s, a)));
+    CDM_DISPATCH_L(L, CDM_DISPATCH_W(W, return (op_mcmc_launch<LG, false, WG>(a, lds, m.queue, m.ncu, s))));
   }
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 // W: the launch's effective register budget (1 for the Rician likelihood).

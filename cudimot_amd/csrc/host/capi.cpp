@@ -173,6 +173,12 @@ int default_group(int method, int nmeas) {
 // a narrow group over a small volume leaves most CUs idle and each voxel's
 // work serial.
 constexpr long long kLaneSlots = 256LL * 4 * 64 * 2;
+// MCMC's floor lies lower, at 1.25 waves per SIMD: four times the lanes cost
+// 1.3 to 1.6 times the work per voxel (the step's serial part runs on every
+// lane).  NODDI_Bingham, 350 jumps, at 4 and 16 lanes: 32,768 voxels 32.5 and
+// 47.7 ms, 16,384 voxels 22.2 and 24.5, 8,192 voxels 22.2 and 13.0;
+// Ball_2_Sticks 30,000 voxels 27.2 and 28.4, 20,480 voxels 26.4 and 20.5.
+constexpr long long kMcmcLaneSlots = 256LL * 4 * 64 * 5 / 4;
 
 // Tuned entry of the nearest measurement count (log ratio), or null.
 const cdm_model::Tuned* tuned_for(const cdm_model* m, int method, int nmeas) {
@@ -193,7 +199,8 @@ int group_for(const cdm_model* m, int method, int nmeas, int nvox) {
   if (m->group[method]) return m->group[method];
   const cdm_model::Tuned* t = tuned_for(m, method, nmeas);
   int L = t ? t->lanes : default_group(method, nmeas);
-  while (nvox > 0 && L < 64 && (long long)nvox * L < kLaneSlots) L *= 4;
+  const long long floor = method == cdm::kMcmc ? kMcmcLaneSlots : kLaneSlots;
+  while (nvox > 0 && L < 64 && (long long)nvox * L < floor) L *= 4;
   return L;
 }
 
@@ -405,6 +412,17 @@ int upload_grid(cdm_model* m) {
   }
   m->grid_dirty = false;
   return 0;
+}
+
+// Compute units of the current device (0 if unknown).
+int device_cus() {
+  int dev = 0, ncu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return ncu;
 }
 
 // MCMC chain state of nvox voxels, followed (256-byte aligned) by the two
@@ -721,17 +739,6 @@ int cdm_model_set_mcmc_blocks(cdm_model* m, int jumps_per_launch, int use_graph)
   return 0;
 }
 
-// Compute units of the current device (0 if unknown).
-static int device_cus() {
-  int dev = 0, ncu = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-    (void)hipGetLastError();
-    return 0;
-  }
-  return ncu;
-}
-
 // Slices of the combinations for a GridSearch whose voxel groups alone
 // leave the GPU mostly idle: enough (at most `most`, at least 64 combinations
 // each) for about 8 blocks per CU; 1 for volumes that fill it.
@@ -889,10 +896,11 @@ size_t mcmc_state_bytes(const cdm_model* m, int nvox, int nmeas, const float* cf
 // jumps_per_launch jumps (0: whole phases), over the chain state at `state`
 // (nvox voxels, their cache rows after it).  use_graph: record a blocked
 // phase into a HIP graph kept by the handle and replayed by later calls.
+// queue: mcmc_queue_ints(nvox) device ints for launches in time slices, or null.
 int run_mcmc(cdm_model* m, int nvox, int nmeas, const float* meas, float* params, const float* cfp, const float* fixp,
              int nburn, int njumps, int sampleevery, int update_proposal, int rician, unsigned long long seed,
-             long long voxel_offset, float* samples, float* tau_samples, void* state, int jumps_per_launch,
-             bool use_graph, hipStream_t s) {
+             long long voxel_offset, float* samples, float* tau_samples, void* state, int* queue,
+             int jumps_per_launch, bool use_graph, hipStream_t s) {
   const int nb = nburn < 1 ? 1 : nburn;  // MCMC.cu:702-703
   const int nsamples = njumps / sampleevery;
   const cdm::Geom g = make_geom(m, nvox, nmeas, meas, cfp, fixp);
@@ -913,6 +921,8 @@ int run_mcmc(cdm_model* m, int nvox, int nmeas, const float* meas, float* params
   ml.upe = sampleevery;
   ml.seed = seed;
   ml.voxel_offset = voxel_offset;
+  ml.queue = queue;
+  ml.ncu = queue ? device_cus() : 0;
   for (int phase = 0; phase < 2; ++phase) {
     const int len = phase == 0 ? nb : njumps;
     const int blk = jumps_per_launch > 0 ? jumps_per_launch : len;
@@ -956,13 +966,16 @@ int mcmc_call(cdm_model* m, int nvox, int nmeas, const float* meas, float* param
               int nburn, int njumps, int sampleevery, int update_proposal, int rician, unsigned long long seed,
               long long voxel_offset, float* samples, float* tau_samples, int jumps_per_launch, bool use_graph,
               hipStream_t s) {
-  int r = ensure_state(m, mcmc_state_bytes(m, nvox, nmeas, cfp, fixp, rician));
+  // the chain state, then the queue of launches in time slices
+  const size_t state_bytes = (mcmc_state_bytes(m, nvox, nmeas, cfp, fixp, rician) + 255) / 256 * 256;
+  int r = ensure_state(m, state_bytes + cdm::mcmc_queue_ints(nvox) * sizeof(int));
   if (r) return r;
   hipError_t e = order_after_last(m, s);
   if (e != hipSuccess) return hip_fail(e, "MCMC stream order");
   if ((e = debug_reset(m, 2, s)) != hipSuccess) return hip_fail(e, "MCMC --debug records");
   r = run_mcmc(m, nvox, nmeas, meas, params, cfp, fixp, nburn, njumps, sampleevery, update_proposal, rician, seed,
-               voxel_offset, samples, tau_samples, m->d_state, jumps_per_launch, use_graph, s);
+               voxel_offset, samples, tau_samples, m->d_state, (int*)((char*)m->d_state + state_bytes),
+               jumps_per_launch, use_graph, s);
   if (r) return r;
   e = note_last(m, s);
   return e == hipSuccess ? 0 : hip_fail(e, "MCMC stream order");
@@ -1001,7 +1014,7 @@ int cdm_mcmc_noalloc(cdm_model* m, int nvox, int nmeas, const float* meas, float
   if (e != hipSuccess) return hip_fail(e, "allocation-free scratch lookup");
   if ((e = debug_reset(m, 2, (hipStream_t)stream)) != hipSuccess) return hip_fail(e, "MCMC --debug records");
   return run_mcmc(m, nvox, nmeas, meas, params, cfp, fixp, nburn, njumps, sampleevery, update_proposal, rician, seed,
-                  voxel_offset, samples, tau_samples, scratch, m->mcmc_block, false, (hipStream_t)stream);
+                  voxel_offset, samples, tau_samples, scratch, nullptr, m->mcmc_block, false, (hipStream_t)stream);
 }
 
 int cdm_predicted_signal(cdm_model* m, int nvox, int nmeas, int nsamples, const float* samples, const float* cfp,

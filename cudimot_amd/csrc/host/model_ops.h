@@ -39,9 +39,17 @@ struct McmcLaunch {
   int recording, update_prop;
   int begin, count, phase_len;
   unsigned jump_offset;
+  int ncu = 0;  // the device's compute units
   unsigned long long seed;
   long long voxel_offset;
+  // device ints for a launch in time slices (mcmc_queue_ints of the voxels;
+  // null: one block per tile)
+  int* queue = nullptr;
 };
+
+// The ticket counter and a count per tile, for the widest group (four voxels a
+// tile).
+inline size_t mcmc_queue_ints(int nvox) { return 16 + ((size_t)nvox + 3) / 4; }
 
 enum Method { kGridSearch = 0, kLevMar = 1, kMcmc = 2, kPredicted = 3, kBicAic = 4 };
 

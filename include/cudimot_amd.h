@@ -78,7 +78,7 @@ int cdm_model_grid(const cdm_model* m, int* grid_params, double* grid);
 /* Voxel-group size (lanes per voxel: 1, 4, 16 or 64) used by a method;
  * 0 restores the automatic choice: the tuned or built-in size for the
  * measurement count, widened for launches over few voxels (nvox x lanes
- * below ~131k lane slots) so that the grid still fills the GPU.  get_group
+ * below ~131k lane slots, MCMC ~82k) so that the grid still fills the GPU.  get_group
  * reports the size a launch of nvox voxels would use (nvox <= 0: no
  * widening). */
 int cdm_model_set_group(cdm_model* m, int method, int lanes);
