@@ -108,7 +108,7 @@ def batch_unit_source(name, model_dirs):
     out = ["// generated: batch unit %s (%s)" % (name, ", ".join(m for m, _ in model_dirs)),
            '#include "abi/functions_gpu.h"', '#include "engine/philox.h"', '#include "engine/wave.h"',
            '#include "engine/packed.h"', '#include "host/model_ops.h"', "#include <algorithm>", "#include <climits>",
-           "#include <cstring>", ""]
+           "#include <cstring>", "#define CDM_BATCH_UNIT", ""]
     for k, (m, d) in enumerate(model_dirs):
         out += ["#undef %s" % x for x in PLUGIN_MACROS]
         out += ["namespace cdm_batch_%s_m%d {" % (name, k),

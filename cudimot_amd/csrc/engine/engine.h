@@ -102,8 +102,15 @@ constexpr int cdm_ntri = cdm::tri_size(NPARAMS);
 //                              fr) (with CDM_MEAS_VOXEL_CACHE also
 //                              Predicted_Signal_MV_Framed and
 //                              Predicted_Signal_MV_Fill_Framed) give the values of
-//                              the plain forms from them.  MCMC keeps them per
-//                              voxel: a step recomputes only those it moves
+//                              the plain forms from them.  The k-th parameter of
+//                              the mask owns an equal run of the entries, the
+//                              k-th.  MCMC keeps them per voxel, a step
+//                              recomputes only those it moves; LM and the FP64
+//                              costs form them once per parameter vector.  For
+//                              LM, Predicted_Signal_Partials_Framed(npar, P, CFP,
+//                              FixP, vc, mc, d, fr) (with CDM_SIGNAL_PARTIALS) or
+//                              Partial_Derivatives_Framed(npar, P, CFP, FixP, d,
+//                              fr) (without CDM_NUMERICAL_MASK)
 //   CDM_GRID_LINEAR b          GridSearch: the signal is a weighted sum of basis
 //                              signals, S = sum_k w_k B_k, and the parameters
 //                              in b enter the weights only
@@ -259,6 +266,72 @@ __device__ __forceinline__ TF cdm_signal(TF* p, TF* cfp, TF* fx, const CDM_F64* 
   return Predicted_Signal(cdm_np, p, cfp, fx);
 #endif
 }
+
+// The index of the k-th parameter in a mask.
+__device__ __forceinline__ int cdm_nth_param(unsigned mask, int k) {
+  int idx = 0, c = 0;
+#pragma unroll
+  for (int b = 0; b < cdm_np; ++b)
+    if ((mask >> b) & 1u) {
+      if (c == k) idx = b;
+      ++c;
+    }
+  return idx;
+}
+
+// Frame values of the parameters p by a group of L lanes: lane k computes the
+// k-th frame parameter's run of entries and hands it to the group.  LM's kernels
+// inlined a sine and cosine pair per angle into every probe and cost, which
+// filled the instruction cache (NODDI_Bingham: 22,500 instructions, 1.1e7
+// instruction fetch misses; with frames 11,600 and 2e5).  Measured, with the
+// transforms over lanes below: NODDI_Bingham, 50,003 voxels of 99 measurements
+// and 8 iterations, 15.2 -> 12.3 ms; NODDI_Watson, 60,000 and 12, 9.3 -> 6.5 ms;
+// Ball_1_Stick, 400 voxels of 64, 160 -> 118 us.
+constexpr int cdm_frame_params = __builtin_popcount(cdm_frame_dep);
+constexpr int cdm_frame_run = cdm_frame_params > 0 ? cdm_nframe / cdm_frame_params : 1;
+static_assert(cdm_frame_params == 0 || cdm_frame_run * cdm_frame_params == cdm_nframe, "equal runs of frame entries");
+template <int L, class TF>
+__device__ __forceinline__ void cdm_frame_g(TF* p, TF* fr, int lane) {
+#ifdef CDM_SIGNAL_FRAME
+  constexpr int rounds = (cdm_frame_params + L - 1) / L;
+#pragma unroll
+  for (int r = 0; r < rounds; ++r) {
+    const int k = min(r * L + lane, cdm_frame_params - 1);
+    TF f[cdm_nframe];
+#pragma unroll
+    for (int e = 0; e < cdm_nframe; ++e) f[e] = (TF)0;
+    Signal_Frame(cdm_np, p, f, cdm_nth_param(cdm_frame_dep, k));
+    TF run[cdm_frame_run];
+#pragma unroll
+    for (int e = 0; e < cdm_frame_run; ++e) {
+      run[e] = (TF)0;
+#pragma unroll
+      for (int q = 0; q < cdm_frame_params; ++q)
+        if (q == k) run[e] = f[q * cdm_frame_run + e];
+    }
+#pragma unroll
+    for (int q = r * L; q < (r + 1) * L && q < cdm_frame_params; ++q)
+#pragma unroll
+      for (int e = 0; e < cdm_frame_run; ++e) fr[q * cdm_frame_run + e] = cdm::Group<L>::bcast(run[e], q - r * L);
+  }
+#else
+  (void)p;
+  (void)fr;
+  (void)lane;
+#endif
+}
+
+// The signal from the frame's values, and the plain form without a frame.
+template <class TF>
+__device__ __forceinline__ TF cdm_signal_fr(TF* p, TF* cfp, TF* fx, const CDM_F64* vc, const CDM_F64* mc, const TF* fr) {
+#ifdef CDM_SIGNAL_FRAME
+  return Predicted_Signal_Framed(cdm_np, p, cfp, fx, vc, mc, fr);
+#else
+  (void)fr;
+  return cdm_signal(p, cfp, fx, vc, mc);
+#endif
+}
+constexpr int cdm_frame_n = cdm_nframe > 0 ? cdm_nframe : 1;
 constexpr int cdm_cfp_max = 16;
 constexpr int cdm_fixp_max = 8;
 constexpr int cdm_block = 256;
@@ -368,8 +441,10 @@ __device__ __forceinline__ double cdm_sse(const cdm_geom& g, const float* s_cfp,
   cdm_cfp_row<TF> row;
   CDM_F64 vc[cdm_vc];
   cdm_prepare_g<L>(p, fx, vc, lane);
+  TF fr[cdm_frame_n];
+  cdm_frame_g<L>(p, fr, lane);
   for (int m = lane; m < g.nmeas; m += L) {
-    const TF s = cdm_signal(p, row.at(s_cfp, m, g.cfp_ts), fx, vc, cdm_mc_row(s_mc, m));
+    const TF s = cdm_signal_fr(p, row.at(s_cfp, m, g.cfp_ts), fx, vc, cdm_mc_row(s_mc, m), fr);
     const TF r = s - (TF)mv[m];
     acc += (double)(r * r);
   }
@@ -1275,70 +1350,124 @@ __device__ __forceinline__ void cdm_minmax_t(double lo, double hi, double p, dou
   t = tan(t) * cdm_lm_speed;
 }
 
-__device__ __forceinline__ void cdm_inv_transform(const cdm_consts& c, double* p, double* t) {
-#pragma unroll
-  for (int i = 0; i < cdm_np; ++i) {
-    const int bt = c.bound_types[i];
-    const double lo = c.bmin[i], hi = c.bmax[i];
-    if (bt == cdm_BMIN) {
-      t[i] = log(p[i] - lo);
-    } else if (bt == cdm_BMAX) {
-      t[i] = log(hi - p[i]);
-    } else if (bt == cdm_BMINMAX) {
-      if (p[i] <= lo + cdm_lm_avoid) p[i] += cdm_lm_avoid;
-      if (p[i] >= hi - cdm_lm_avoid) p[i] -= cdm_lm_avoid;
-      cdm_minmax_t(lo, hi, p[i], t[i]);
-    } else {
-      t[i] = p[i];
-    }
+// One parameter's transforms (bound type bt, bounds lo, hi).  They name their
+// fused multiply-adds, so that every kernel that inlines them rounds alike.
+__device__ __forceinline__ void cdm_inv_transform1(int bt, double lo, double hi, double& p, double& t) {
+  if (bt == cdm_BMIN) {
+    t = log(p - lo);
+  } else if (bt == cdm_BMAX) {
+    t = log(hi - p);
+  } else if (bt == cdm_BMINMAX) {
+    if (p <= lo + cdm_lm_avoid) p += cdm_lm_avoid;
+    if (p >= hi - cdm_lm_avoid) p -= cdm_lm_avoid;
+    cdm_minmax_t(lo, hi, p, t);
+  } else {
+    t = p;
   }
 }
 
-__device__ __forceinline__ void cdm_transform(const cdm_consts& c, double* p, double* t) {
-#pragma unroll
-  for (int i = 0; i < cdm_np; ++i) {
-    const int bt = c.bound_types[i];
-    const double lo = c.bmin[i], hi = c.bmax[i];
-    if (bt == cdm_BMIN) {
-      p[i] = exp(t[i]) + lo;
-    } else if (bt == cdm_BMAX) {
-      p[i] = hi - exp(t[i]);
-    } else if (bt == cdm_BMINMAX) {
-      double x = (hi - lo) / 2.0;
-      x *= atan(t[i] / cdm_lm_speed);
-      x *= cdm_lm_twodivpi;
-      x += (lo + hi) / 2.0;
-      if (x <= lo + cdm_lm_avoid) {
-        x += cdm_lm_avoid;
-        cdm_minmax_t(lo, hi, x, t[i]);
-      }
-      if (x >= hi - cdm_lm_avoid) {
-        x -= cdm_lm_avoid;
-        cdm_minmax_t(lo, hi, x, t[i]);
-      }
-      p[i] = x;
-    } else {
-      p[i] = t[i];
+__device__ __forceinline__ void cdm_transform1(int bt, double lo, double hi, double& p, double& t) {
+  if (bt == cdm_BMIN) {
+    p = exp(t) + lo;
+  } else if (bt == cdm_BMAX) {
+    p = hi - exp(t);
+  } else if (bt == cdm_BMINMAX) {
+    const double half = ((hi - lo) / 2.0) * atan(t / cdm_lm_speed);
+    double x = fma(half, cdm_lm_twodivpi, (lo + hi) / 2.0);
+    if (x <= lo + cdm_lm_avoid) {
+      x += cdm_lm_avoid;
+      cdm_minmax_t(lo, hi, x, t);
     }
+    if (x >= hi - cdm_lm_avoid) {
+      x -= cdm_lm_avoid;
+      cdm_minmax_t(lo, hi, x, t);
+    }
+    p = x;
+  } else {
+    p = t;
   }
 }
 
 // d(param)/d(transformed param), Levenberg_Marquardt.cu:120-135.
-__device__ __forceinline__ void cdm_dtransform(const cdm_consts& c, const double* t, double* d) {
+__device__ __forceinline__ double cdm_dtransform1(int bt, float lo, float hi, double t) {
+  if (bt == cdm_BMIN) return exp(t);
+  if (bt == cdm_BMAX) return -exp(t);
+  if (bt == cdm_BMINMAX) {
+    const float span = hi - lo;  // float difference, as the reference
+    return (span / 2.0) * cdm_lm_twodivpi * (cdm_lm_speed / fma(t, t, cdm_lm_speed * cdm_lm_speed));
+  }
+  return 1.0;
+}
+
+// The transforms of all parameters by a group of L lanes: lane i (i + L, ...)
+// transforms parameter i and hands it to the group, so the exponentials and
+// arctangents of all parameters issue once instead of one after the other.  One
+// lane per voxel does them in turn, and so do the batch units, whose kernels
+// run out of registers already (the spread form compiled there to a kernel that
+// rejected every step of the 14-parameter plug-in).  Same values either way.
+// DiffusionTensor, the same kernel otherwise: 1.27 -> 0.99 ms.
+#ifdef CDM_BATCH_UNIT
+constexpr bool cdm_lane_transforms = false;
+#else
+constexpr bool cdm_lane_transforms = true;
+#endif
+template <int L, class F>
+__device__ __forceinline__ void cdm_per_param(const cdm_consts& c, double* p, double* t, int lane, F f) {
+  if constexpr (L == 1 || !cdm_lane_transforms) {
 #pragma unroll
-  for (int i = 0; i < cdm_np; ++i) {
-    const int bt = c.bound_types[i];
-    if (bt == cdm_BMIN) {
-      d[i] = exp(t[i]);
-    } else if (bt == cdm_BMAX) {
-      d[i] = -exp(t[i]);
-    } else if (bt == cdm_BMINMAX) {
-      const float span = c.bmax[i] - c.bmin[i];  // float difference, as the reference
-      d[i] = (span / 2.0) * cdm_lm_twodivpi * (cdm_lm_speed / (cdm_lm_speed * cdm_lm_speed + t[i] * t[i]));
-    } else {
-      d[i] = 1.0;
+    for (int i = 0; i < cdm_np; ++i) f(c.bound_types[i], c.bmin[i], c.bmax[i], p[i], t[i]);
+  } else {
+#pragma unroll
+    for (int r = 0; r < (cdm_np + L - 1) / L; ++r) {
+      const int mine = r * L + lane;
+      int bt = cdm_NOBOUNDS;
+      float lo = 0.f, hi = 0.f;
+      double pm = 0.0, tm = 0.0;
+#pragma unroll
+      for (int i = r * L; i < (r + 1) * L && i < cdm_np; ++i)
+        if (i == mine) {
+          bt = c.bound_types[i];
+          lo = c.bmin[i];
+          hi = c.bmax[i];
+          pm = p[i];
+          tm = t[i];
+        }
+      f(bt, lo, hi, pm, tm);
+#pragma unroll
+      for (int i = r * L; i < (r + 1) * L && i < cdm_np; ++i) {
+        p[i] = cdm::Group<L>::bcast(pm, i - r * L);
+        t[i] = cdm::Group<L>::bcast(tm, i - r * L);
+      }
     }
   }
+}
+
+template <int L>
+__device__ __forceinline__ void cdm_inv_transform(const cdm_consts& c, double* p, double* t, int lane) {
+#pragma unroll
+  for (int i = 0; i < cdm_np; ++i) t[i] = 0.0;
+  cdm_per_param<L>(c, p, t, lane, [](int bt, float lo, float hi, double& pi, double& ti) {
+    cdm_inv_transform1(bt, lo, hi, pi, ti);
+  });
+}
+template <int L>
+__device__ __forceinline__ void cdm_transform(const cdm_consts& c, double* p, double* t, int lane) {
+  cdm_per_param<L>(c, p, t, lane, [](int bt, float lo, float hi, double& pi, double& ti) {
+    cdm_transform1(bt, lo, hi, pi, ti);
+  });
+}
+// d[i] of every parameter.
+template <int L>
+__device__ __forceinline__ void cdm_dtransform(const cdm_consts& c, const double* t, double* d, int lane) {
+  double tt[cdm_np];
+#pragma unroll
+  for (int i = 0; i < cdm_np; ++i) {
+    tt[i] = t[i];
+    d[i] = 0.0;
+  }
+  cdm_per_param<L>(c, d, tt, lane, [](int bt, float lo, float hi, double& di, double& ti) {
+    di = cdm_dtransform1(bt, lo, hi, ti);
+  });
 }
 
 // Signal and Jacobian at one measurement.  With CDM_NUMERICAL_MASK the
@@ -1358,6 +1487,11 @@ constexpr bool cdm_jac_keep_probes =
 template <class TJ>
 struct cdm_jacobian_setup {
   CDM_F64 vc0[cdm_vc];
+  TJ fr0[cdm_frame_n];
+#if defined(CDM_NUMERICAL_MASK) && defined(CDM_SIGNAL_FRAME)
+  // the moved runs of the probes p_i + h/2 and p_i + h/2 - 2 (h/2)
+  TJ frp[cdm_frame_params][cdm_frame_run], frm[cdm_frame_params][cdm_frame_run];
+#endif
 #ifdef CDM_NUMERICAL_MASK
   CDM_F64 vcp[cdm_np][cdm_vc], vcm[cdm_np][cdm_vc];  // unused (removed) without cdm_jac_keep_probes
   TJ h[cdm_np];
@@ -1392,6 +1526,67 @@ struct cdm_jacobian_setup {
     return vc0;
   }
 #endif
+  // Frames at p and the runs its probes move: entry set k of 3 (p, upper, lower
+  // probe of a frame parameter) on its own lane.
+  template <int L>
+  __device__ __forceinline__ void init_frames(TJ* p, int lane) {
+#ifdef CDM_SIGNAL_FRAME
+#ifdef CDM_NUMERICAL_MASK
+    static_assert((cdm_frame_dep & ~(unsigned)(CDM_NUMERICAL_MASK)) == 0, "frame parameters have central differences");
+    constexpr int T = 3 * cdm_frame_params, rounds = (T + L - 1) / L;
+    TJ run[rounds][cdm_frame_run];
+#pragma unroll
+    for (int r = 0; r < rounds; ++r) {
+      const int t = min(lane + r * L, T - 1), k = t / 3, side = t - 3 * k;
+      const int i = cdm_nth_param(cdm_frame_dep, k);
+      TJ q[cdm_np], f[cdm_nframe];
+#pragma unroll
+      for (int j = 0; j < cdm_np; ++j) {
+        const TJ up = p[j] + h[j] * (TJ)0.5;
+        const TJ dn = up - (TJ)2 * (h[j] * (TJ)0.5);
+        q[j] = j != i || side == 0 ? p[j] : side == 1 ? up : dn;
+      }
+#pragma unroll
+      for (int e = 0; e < cdm_nframe; ++e) f[e] = (TJ)0;
+      Signal_Frame(cdm_np, q, f, i);
+#pragma unroll
+      for (int e = 0; e < cdm_frame_run; ++e) {
+        run[r][e] = (TJ)0;
+#pragma unroll
+        for (int j = 0; j < cdm_frame_params; ++j)
+          if (j == k) run[r][e] = f[j * cdm_frame_run + e];
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < cdm_frame_params; ++k)
+#pragma unroll
+      for (int e = 0; e < cdm_frame_run; ++e) {
+        fr0[k * cdm_frame_run + e] = cdm::Group<L>::bcast(run[(3 * k) / L][e], (3 * k) % L);
+        frp[k][e] = cdm::Group<L>::bcast(run[(3 * k + 1) / L][e], (3 * k + 1) % L);
+        frm[k][e] = cdm::Group<L>::bcast(run[(3 * k + 2) / L][e], (3 * k + 2) % L);
+      }
+#else
+    cdm_frame_g<L>(p, fr0, lane);
+#endif
+#endif
+  }
+#if defined(CDM_NUMERICAL_MASK) && defined(CDM_SIGNAL_FRAME)
+  // The frame of a probe of parameter i (side 0 upper, 1 lower).
+  __device__ __forceinline__ void probe_frame(int i, int side, TJ* fr) const {
+#pragma unroll
+    for (int e = 0; e < cdm_nframe; ++e) fr[e] = fr0[e];
+    int k = 0;
+#pragma unroll
+    for (int b = 0; b < cdm_np; ++b) {
+      if (!((cdm_frame_dep >> b) & 1u)) continue;
+      if (b == i) {
+#pragma unroll
+        for (int e = 0; e < cdm_frame_run; ++e) fr[k * cdm_frame_run + e] = side == 0 ? frp[k][e] : frm[k][e];
+      }
+      ++k;
+    }
+  }
+#endif
   // Voxel caches at p and at every dependent probe.  When the group has at
   // least as many lanes as caches, lane j computes cache j and the group
   // exchanges them, instead of every lane computing all of them.
@@ -1405,6 +1600,7 @@ struct cdm_jacobian_setup {
       hi = min_gpu(max_gpu(hi, (TJ)::cdm_fd_step<TJ>::lo), (TJ)::cdm_fd_step<TJ>::hi);
       h[i] = hi;
     }
+    init_frames<L>(p, lane);
     constexpr int njobs = 1 + 2 * __builtin_popcount(CDM_NUMERICAL_MASK & cdm_vc_dep);
     if constexpr (!cdm_jac_keep_probes) {
       cdm_prepare_g<L>(p, fx, vc0, lane);
@@ -1481,6 +1677,7 @@ struct cdm_jacobian_setup {
       p[i] = keep;
     }
 #else
+    init_frames<L>(p, lane);
     (void)lane;
     cdm_prepare(p, fx, vc0);
 #endif
@@ -1491,12 +1688,29 @@ struct cdm_jacobian_setup {
 #else
 #pragma unroll
     for (int i = 0; i < cdm_np; ++i) d[i] = (TJ)0;
-    const TJ s = cdm_signal(p, cm, fx, vc0, mc);
+    const TJ s = cdm_signal_fr(p, cm, fx, vc0, mc, fr0);
+#ifdef CDM_SIGNAL_FRAME
+    Partial_Derivatives_Framed(cdm_np, p, cm, fx, d, fr0);
+#else
     Partial_Derivatives(cdm_np, p, cm, fx, d);
+#endif
     return s;
 #endif
   }
 #ifdef CDM_NUMERICAL_MASK
+  // The signal at the probe p of parameter i on side `side`.
+  __device__ __forceinline__ TJ probe_signal(int i, int side, TJ* p, TJ* cm, TJ* fx, const CDM_F64* vc,
+                                             const CDM_F64* mc) const {
+#ifdef CDM_SIGNAL_FRAME
+    TJ fr[cdm_nframe];
+    probe_frame(i, side, fr);
+    return Predicted_Signal_Framed(cdm_np, p, cm, fx, vc, mc, fr);
+#else
+    (void)i;
+    (void)side;
+    return cdm_signal(p, cm, fx, vc, mc);
+#endif
+  }
   // eval restricted to the central differences of the parameters in PROBES
   // (a subset of CDM_NUMERICAL_MASK), with the signal and the analytic
   // entries when SIGNAL (0 is returned otherwise); each entry is eval's.
@@ -1506,7 +1720,9 @@ struct cdm_jacobian_setup {
     for (int i = 0; i < cdm_np; ++i) d[i] = (TJ)0;
     TJ s = (TJ)0;
     if constexpr (SIGNAL) {
-#ifdef CDM_SIGNAL_PARTIALS
+#if defined(CDM_SIGNAL_PARTIALS) && defined(CDM_SIGNAL_FRAME)
+      s = Predicted_Signal_Partials_Framed(cdm_np, p, cm, fx, vc0, mc, d, fr0);
+#elif defined(CDM_SIGNAL_PARTIALS)
       s = Predicted_Signal_Partials_Cached(cdm_np, p, cm, fx, vc0, mc, d);
 #else
       s = cdm_signal(p, cm, fx, vc0, mc);
@@ -1521,9 +1737,9 @@ struct cdm_jacobian_setup {
       TJ up, dn;
       if constexpr (cdm_jac_keep_probes) {
         p[i] += h[i] * (TJ)0.5;
-        up = cdm_signal(p, cm, fx, dep ? vcp[i] : vc0, mc);
+        up = probe_signal(i, 0, p, cm, fx, dep ? vcp[i] : vc0, mc);
         p[i] -= (TJ)2 * (h[i] * (TJ)0.5);
-        dn = cdm_signal(p, cm, fx, dep ? vcm[i] : vc0, mc);
+        dn = probe_signal(i, 1, p, cm, fx, dep ? vcm[i] : vc0, mc);
       } else {
         CDM_F64 vq[cdm_vc];
         p[i] += h[i] * (TJ)0.5;
@@ -1872,7 +2088,7 @@ __device__ __forceinline__ void cdm_levmar_voxel(const cdm_lm_args& a, int marqu
   double p[cdm_np], t[cdm_np];
 #pragma unroll
   for (int i = 0; i < cdm_np; ++i) p[i] = a.params[(size_t)v * cdm_np + i];
-  cdm_inv_transform(a.c, p, t);
+  cdm_inv_transform<L>(a.c, p, t, lane);
 
   double fxd[cdm_fixp_max];
 #pragma unroll
@@ -1894,7 +2110,7 @@ __device__ __forceinline__ void cdm_levmar_voxel(const cdm_lm_args& a, int marqu
   while (!(success && iter++ >= a.max_iters)) {
     if (success) {
       double dt[cdm_np];
-      cdm_dtransform(a.c, t, dt);
+      cdm_dtransform<L>(a.c, t, dt, lane);
       cdm_jt dtf[cdm_np], pj[cdm_np], fxj[cdm_fixp_max];
 #pragma unroll
       for (int i = 0; i < cdm_np; ++i) {
@@ -2082,7 +2298,7 @@ __device__ __forceinline__ void cdm_levmar_voxel(const cdm_lm_args& a, int marqu
     double tn[cdm_np];
 #pragma unroll
     for (int i = 0; i < cdm_np; ++i) tn[i] = t[i] - step[i];
-    cdm_transform(a.c, p, tn);
+    cdm_transform<L>(a.c, p, tn, lane);
     const double ncf = cdm_sse<L>(a.g, s_cfp, s_mc, mv, p, fxd, lane);
     bool end = false;
     success = ncf < pcf;
@@ -2098,7 +2314,7 @@ __device__ __forceinline__ void cdm_levmar_voxel(const cdm_lm_args& a, int marqu
       olambda = lambda;
       lambda = lambda * 10.0;
       if (lambda > cdm_lm_ltol) end = true;
-      cdm_transform(a.c, p, t);
+      cdm_transform<L>(a.c, p, t, lane);
     }
     if (dbg) {
       cdm_dbg_record(a.c, 1, dbg_slot, (double)dbg_slot, success ? pcf : ncf, lambda, success ? 1.0 : 0.0, p);

@@ -8,14 +8,20 @@
 // below what the float rounding of the argument b d (g.n)^2 itself
 // brings); double-precision evaluations use the exact exp.
 
-MACRO void b1s_geometry(const T* P, const T* CFP, T& gn, T& dgn_dth, T& dgn_dph) {
-  T st, ct, sp, cp;
-  tsincos(P[3], &st, &ct);
-  tsincos(P[4], &sp, &cp);
+// tr: sine and cosine of th and of ph.
+MACRO void b1s_directions(const T* CFP, const T* tr, T& gn, T& dgn_dth, T& dgn_dph) {
+  const T st = tr[0], ct = tr[1], sp = tr[2], cp = tr[3];
   const T gxy = CFP[0] * cp + CFP[1] * sp;  // g projected on the stick azimuth
   gn = st * gxy + CFP[2] * ct;
   dgn_dth = ct * gxy - st * CFP[2];
   dgn_dph = st * (CFP[1] * cp - CFP[0] * sp);
+}
+
+MACRO void b1s_geometry(const T* P, const T* CFP, T& gn, T& dgn_dth, T& dgn_dph) {
+  T tr[4];
+  tsincos(P[3], &tr[0], &tr[1]);
+  tsincos(P[4], &tr[2], &tr[3]);
+  b1s_directions(CFP, tr, gn, dgn_dth, dgn_dph);
 }
 
 MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
@@ -108,9 +114,9 @@ MACRO void Grid_Weights(int npar, T* P, T* FixP, T* w) {
 
 MACRO bool ConstraintsMCMC(int npar, T* P) { return true; }
 
-MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {
+MACRO void Partial_Derivatives_Framed(int npar, T* P, T* CFP, T* FixP, T* derivatives, const T* fr) {
   T gn, dth, dph;
-  b1s_geometry(P, CFP, gn, dth, dph);
+  b1s_directions(CFP, fr, gn, dth, dph);
   const T bd = CFP[3] * P[1];
   const T ball = texp_fast(-bd);
   const T stick = texp_fast(-bd * gn * gn);
@@ -121,6 +127,13 @@ MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) 
   const T common = -(T)2 * P[0] * bd * f * gn * stick;  // dS/d(gn) / ... chain factor
   derivatives[3] = common * dth;
   derivatives[4] = common * dph;
+}
+
+MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {
+  T fr[4];
+  tsincos(P[3], &fr[0], &fr[1]);
+  tsincos(P[4], &fr[2], &fr[3]);
+  Partial_Derivatives_Framed(npar, P, CFP, FixP, derivatives, fr);
 }
 
 MACRO void FixConstraintsLM(int npar, T* P) {}

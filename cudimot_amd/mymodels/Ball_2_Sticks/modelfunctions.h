@@ -13,14 +13,20 @@
 // below what the float rounding of the argument b d (g.n)^2 itself
 // brings); double-precision evaluations use the exact exp.
 
-MACRO void b2s_stick(const T* CFP, T th, T ph, T& gn, T& dth, T& dph) {
-  T st, ct, sp, cp;
-  tsincos(th, &st, &ct);
-  tsincos(ph, &sp, &cp);
+// tr: sine and cosine of th and of ph.
+MACRO void b2s_directions(const T* CFP, const T* tr, T& gn, T& dth, T& dph) {
+  const T st = tr[0], ct = tr[1], sp = tr[2], cp = tr[3];
   const T gxy = CFP[0] * cp + CFP[1] * sp;
   gn = st * gxy + CFP[2] * ct;
   dth = ct * gxy - st * CFP[2];
   dph = st * (CFP[1] * cp - CFP[0] * sp);
+}
+
+MACRO void b2s_stick(const T* CFP, T th, T ph, T& gn, T& dth, T& dph) {
+  T tr[4];
+  tsincos(th, &tr[0], &tr[1]);
+  tsincos(ph, &tr[2], &tr[3]);
+  b2s_directions(CFP, tr, gn, dth, dph);
 }
 
 MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
@@ -121,10 +127,10 @@ MACRO void Grid_Weights(int npar, T* P, T* FixP, T* w) {
 
 MACRO bool ConstraintsMCMC(int npar, T* P) { return !(P[2] < P[5]); }
 
-MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {
+MACRO void Partial_Derivatives_Framed(int npar, T* P, T* CFP, T* FixP, T* derivatives, const T* fr) {
   T g1, d1th, d1ph, g2, d2th, d2ph;
-  b2s_stick(CFP, P[3], P[4], g1, d1th, d1ph);
-  b2s_stick(CFP, P[6], P[7], g2, d2th, d2ph);
+  b2s_directions(CFP, fr, g1, d1th, d1ph);
+  b2s_directions(CFP, fr + 4, g2, d2th, d2ph);
   const T bd = CFP[3] * P[1];
   const T ball = texp_fast(-bd);
   const T s1 = texp_fast(-bd * g1 * g1);
@@ -144,6 +150,15 @@ MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) 
 #else
   derivatives[7] = c2 * d2th;
 #endif
+}
+
+MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {
+  T fr[8];
+  tsincos(P[3], &fr[0], &fr[1]);
+  tsincos(P[4], &fr[2], &fr[3]);
+  tsincos(P[6], &fr[4], &fr[5]);
+  tsincos(P[7], &fr[6], &fr[7]);
+  Partial_Derivatives_Framed(npar, P, CFP, FixP, derivatives, fr);
 }
 
 // After LM: keep the larger stick first (swap f, th, ph of the two sticks).

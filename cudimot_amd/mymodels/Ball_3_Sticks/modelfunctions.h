@@ -8,14 +8,20 @@
 // below what the float rounding of the argument b d (g.n)^2 itself
 // brings); double-precision evaluations use the exact exp.
 
-MACRO void b3s_stick(const T* CFP, T th, T ph, T& gn, T& dth, T& dph) {
-  T st, ct, sp, cp;
-  tsincos(th, &st, &ct);
-  tsincos(ph, &sp, &cp);
+// tr: sine and cosine of th and of ph.
+MACRO void b3s_directions(const T* CFP, const T* tr, T& gn, T& dth, T& dph) {
+  const T st = tr[0], ct = tr[1], sp = tr[2], cp = tr[3];
   const T gxy = CFP[0] * cp + CFP[1] * sp;
   gn = st * gxy + CFP[2] * ct;
   dth = ct * gxy - st * CFP[2];
   dph = st * (CFP[1] * cp - CFP[0] * sp);
+}
+
+MACRO void b3s_stick(const T* CFP, T th, T ph, T& gn, T& dth, T& dph) {
+  T tr[4];
+  tsincos(th, &tr[0], &tr[1]);
+  tsincos(ph, &tr[2], &tr[3]);
+  b3s_directions(CFP, tr, gn, dth, dph);
 }
 
 MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
@@ -123,7 +129,7 @@ MACRO void Grid_Weights(int npar, T* P, T* FixP, T* w) {
 
 MACRO bool ConstraintsMCMC(int npar, T* P) { return !(P[2] < P[5]) && !(P[5] < P[8]); }
 
-MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {
+MACRO void Partial_Derivatives_Framed(int npar, T* P, T* CFP, T* FixP, T* derivatives, const T* fr) {
   const T bd = CFP[3] * P[1];
   const T ball = texp_fast(-bd);
   const T fb = (T)1 - P[2] - P[5] - P[8];
@@ -131,7 +137,7 @@ MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) 
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     T g, dth, dph;
-    b3s_stick(CFP, P[3 + 3 * k], P[4 + 3 * k], g, dth, dph);
+    b3s_directions(CFP, fr + 4 * k, g, dth, dph);
     const T sk = texp_fast(-bd * g * g);
     const T fk = P[2 + 3 * k];
     mix += fk * sk;
@@ -143,6 +149,16 @@ MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) 
   }
   derivatives[0] = mix;
   derivatives[1] = -P[0] * CFP[3] * dmix;
+}
+
+MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {
+  T fr[12];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    tsincos(P[3 + 3 * k], &fr[4 * k], &fr[4 * k + 1]);
+    tsincos(P[4 + 3 * k], &fr[4 * k + 2], &fr[4 * k + 3]);
+  }
+  Partial_Derivatives_Framed(npar, P, CFP, FixP, derivatives, fr);
 }
 
 // After LM: order the sticks by decreasing fraction.

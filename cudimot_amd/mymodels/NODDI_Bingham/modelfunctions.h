@@ -246,6 +246,24 @@ MACRO T Predicted_Signal_Partials_Cached(int npar, T* P, T* CFP, T* FixP, const 
   return FixP[0] * (((T)1 - P[0]) * fan + P[0] * iso);
 }
 
+MACRO T Predicted_Signal_Partials_Framed(int npar, T* P, T* CFP, T* FixP, const CDM_F64* vc, const CDM_F64* mc,
+                                         T* derivatives, const T* fr) {
+  bingham_fan f;
+  f.lnc4 = vc[0];
+  f.dpar = vc[1];
+  f.dperp1 = vc[2];
+  f.dperp2 = vc[3];
+  T gx, gy, gn;
+  bingham_trig_local(fr, CFP, gx, gy, gn);
+  const T e = bingham_fan_extra_local(gx, gy, gn, CFP[3], f);
+  const T i = bingham_fan_intra_local(P[2], P[3], gx, gy, gn, CFP[3], f);
+  const T fan = ((T)1 - P[1]) * e + P[1] * i;
+  const T iso = (T)mc[0];
+  derivatives[0] = FixP[0] * (iso - fan);
+  derivatives[1] = FixP[0] * ((T)1 - P[0]) * (i - e);
+  return FixP[0] * (((T)1 - P[0]) * fan + P[0] * iso);
+}
+
 MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {
   CDM_F64 vc[4], mc[1];
   Voxel_Cache(npar, P, FixP, vc);

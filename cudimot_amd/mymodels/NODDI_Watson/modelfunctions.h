@@ -189,6 +189,16 @@ MACRO T Predicted_Signal_Partials_Cached(int npar, T* P, T* CFP, T* FixP, const 
   return FixP[0] * (((T)1 - P[0]) * aniso + P[0] * (T)mc[7]);
 }
 
+MACRO T Predicted_Signal_Partials_Framed(int npar, T* P, T* CFP, T* FixP, const CDM_F64* vc, const CDM_F64* mc,
+                                         T* derivatives, const T* fr) {
+  T extra, intra;
+  watson_parts_of(fr, P, CFP, vc, mc, extra, intra);
+  const T aniso = ((T)1 - P[1]) * extra + P[1] * intra;
+  derivatives[0] = FixP[0] * ((T)mc[7] - aniso);
+  derivatives[1] = FixP[0] * ((T)1 - P[0]) * (intra - extra);
+  return FixP[0] * (((T)1 - P[0]) * aniso + P[0] * (T)mc[7]);
+}
+
 MACRO void Partial_Derivatives(int npar, T* P, T* CFP, T* FixP, T* derivatives) {
   CDM_F64 vc[9], mc[8];
   Voxel_Cache(npar, P, FixP, vc);
