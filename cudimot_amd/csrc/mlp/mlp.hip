@@ -39,6 +39,7 @@ namespace {
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kMaxHead = 16;
@@ -376,12 +377,7 @@ __global__ void __launch_bounds__(kLossBlock) loss_kernel(int rows, int n_out, i
 // Raw outputs -> model parameters, entries in order (a ratio entry reads the
 // already-decoded parameter it refers to).  Parameters without an entry keep
 // their value.
-__global__ void decode_kernel(int n, int npad, const float* __restrict__ out, Head h, int nparams,
-                              float* __restrict__ params) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
-  const float* o = out + (size_t)v * npad;
-  float* p = params + (size_t)v * nparams;
+__device__ __forceinline__ void decode_row(const Head& h, const float* o, float* p) {
   for (int j = 0; j < h.n; ++j) {
     const cdm_head_entry& e = h.e[j];
     const int a = h.out_index[j];
@@ -401,6 +397,141 @@ __global__ void decode_kernel(int n, int npad, const float* __restrict__ out, He
       p[e.param] = fminf(fmaxf(x, e.vmin), e.vmax);
     }
   }
+}
+
+__global__ void decode_kernel(int n, int npad, const float* __restrict__ out, Head h, int nparams,
+                              float* __restrict__ params) {
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v >= n) return;
+  decode_row(h, out + (size_t)v * npad, params + (size_t)v * nparams);
+}
+
+// ------------------------------------------------------------- inference
+// Inference in one launch: a block carries 64 rows through every layer, its
+// activations in LDS.  Wave t has unit tile t (32 units) of each layer for both
+// halves of the rows; its weights come straight from L2, each element used
+// twice.  The products run transposed, C = W H^T (W the A operand), so that a
+// lane's accumulators are four runs of four consecutive units of one row, 8-byte
+// stores.  Each product is the same MFMA over the same K order as the
+// layer-by-layer form, so the outputs are the same bits.
+//   Bound by the GELU: 768 erff a row for three layers of 256, about 0.45 ms of
+// VALU issue for 500k rows.  One erff is a chain of dependent instructions, so
+// the kernel wants waves: at most 128 registers, four waves per SIMD (a form
+// with the activations in registers, 231 of them, took 0.69 ms; six waves per
+// SIMD 0.54, but 45 us instead of 42 up to 16,000 rows).  Measured, 500k rows of
+// 99 measurements: 1.52 -> 0.57 ms (the layer-by-layer form moves 270 MB of
+// activations per 65,536 rows); 1 row 34 -> 33 us, 1,000 rows 45 -> 42, 8,000
+// 60 -> 43: taken at any size.
+constexpr int kInferRows = 64;
+constexpr int kInferK = 256;                // most inputs or units of a layer
+constexpr int kInferWaves = kInferK / 32;   // one per unit tile
+constexpr int kInferStride = kInferK + 8;   // bf16 per LDS row: 16 bytes of padding spread the rows over the banks
+
+struct InferLayer {
+  const bf16* w;     // [32 tiles][16 steps]
+  const float* b;    // [32 tiles]
+  int tiles, steps;  // 32-unit tiles, K steps of 16 inputs
+};
+struct InferNet {
+  int n_layers, n_out;
+  InferLayer L[kMaxLayers];
+};
+
+template <int STEPS>
+__device__ __forceinline__ void infer_products(const bf16* w, const bf16* h, f32x16& lo, f32x16& hi) {
+  bf16x8 a[STEPS];
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) a[u] = *(const bf16x8*)(w + 16 * u);
+#pragma unroll
+  for (int u = 0; u < STEPS; ++u) {
+    lo = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], *(const bf16x8*)(h + 16 * u), lo, 0, 0, 0);
+    hi = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], *(const bf16x8*)(h + 32 * kInferStride + 16 * u), hi, 0, 0, 0);
+  }
+}
+
+__global__ void __launch_bounds__(64 * kInferWaves, 4)
+    infer_kernel(InferNet net, Head head, int n, int nmeas, const float* __restrict__ meas,
+                 const float* __restrict__ scale, float* __restrict__ out_raw, int nparams,
+                 float* __restrict__ params) {
+  __shared__ __align__(16) bf16 s_h[kInferRows * kInferStride];
+  __shared__ float s_out[kInferRows][33];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 31, half = lane >> 5;
+  const long long row0 = (long long)blockIdx.x * kInferRows;
+  const int live = (int)min((long long)n - row0, (long long)kInferRows);
+  // the inputs: meas / scale, zero past the live rows and columns
+  const int kpad = 16 * net.L[0].steps;
+  for (int c = lane; c < kpad; c += 64) {
+#pragma unroll
+    for (int k = 0; k < kInferRows / kInferWaves; ++k) {
+      const int row = wave * (kInferRows / kInferWaves) + k;
+      float v = 0.0f;
+      if (row < live && c < nmeas) v = meas[(size_t)(row0 + row) * nmeas + c] / (scale ? scale[row0 + row] : 1.0f);
+      s_h[row * kInferStride + c] = (bf16)v;
+    }
+  }
+  __syncthreads();
+  for (int l = 0; l < net.n_layers; ++l) {
+    const int steps = net.L[l].steps;
+    const bool last = l + 1 == net.n_layers, mine = wave < net.L[l].tiles;
+    f32x16 acc[2] = {};
+    if (mine) {
+      const bf16* h = s_h + r * kInferStride + 8 * half;
+      const bf16* w = net.L[l].w + (size_t)(32 * wave + r) * (16 * steps) + 8 * half;
+      // steps is even and at most 16
+      if (steps & 2) infer_products<2>(w, h, acc[0], acc[1]);
+      if (steps & 4) infer_products<4>(w + 16 * (steps & 2), h + 16 * (steps & 2), acc[0], acc[1]);
+      for (int u = steps & 6; u < steps; u += 8) infer_products<8>(w + 16 * u, h + 16 * u, acc[0], acc[1]);
+      const float* b = net.L[l].b + 32 * wave + 4 * half;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 bias = *(const f32x4*)(b + 8 * g);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[j][4 * g + i] += bias[i];
+      }
+    }
+    if (last) {
+      if (mine) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s_out[32 * j + r][8 * g + 4 * half + i] = acc[j][4 * g + i];
+      }
+      break;
+    }
+    bf16x4 y[2][4] = {};
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (32 * j >= live) continue;  // a short block: no rows in the upper half
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) y[j][g][i] = (bf16)gelu(acc[j][4 * g + i]);
+      }
+    }
+    __syncthreads();  // every wave has read this layer's inputs
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *(bf16x4*)(s_h + (32 * j + r) * kInferStride + 32 * wave + 8 * g + 4 * half) = y[j][g];
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  if (out_raw)
+    for (int i = threadIdx.x; i < live * net.n_out; i += 64 * kInferWaves) {
+      const int k = i / net.n_out;
+      out_raw[(size_t)row0 * net.n_out + i] = s_out[k][i - k * net.n_out];
+    }
+  if (params && (int)threadIdx.x < live)
+    decode_row(head, s_out[threadIdx.x], params + (size_t)(row0 + threadIdx.x) * nparams);
 }
 
 // Adam over weight matrices [nrow][ncol] (padded storage, live region
@@ -837,6 +968,18 @@ AdamStep adam_step_args(cdm_mlp* m, float lr, const StepArgs* tab, int* ctr) {
 // caller's) or straight into the decode step.
 int infer(cdm_mlp* m, int n, int nmeas, const float* meas, const float* scale, float* out_raw, int nparams,
           float* params, hipStream_t s) {
+  // one launch when a layer's units are at most the waves' tiles
+  if (m->width <= kInferK && m->kpad <= kInferK) {
+    InferNet net;
+    std::memset(&net, 0, sizeof(net));
+    net.n_layers = m->depth + 1;
+    net.n_out = m->n_out;
+    for (int l = 0; l <= m->depth; ++l) net.L[l] = {m->wbf[l], m->b[l], m->rows[l] / 32, m->cols[l] / 16};
+    hipLaunchKernelGGL(infer_kernel, grid1(n, kInferRows), dim3(64 * kInferWaves), 0, s, net, m->head, n, nmeas, meas,
+                       scale, out_raw, nparams, params);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : hip_err(e, "network inference launch");
+  }
   int r = ensure_infer(m);
   if (r) return r;
   for (int first = 0; first < n; first += kInferChunk) {

@@ -1,0 +1,48 @@
+"""Network inference in one launch (layers of at most 256 inputs and units)
+against the layer-by-layer form, at the edges of its blocks of 64 rows, of the
+64-column input runs and of the 32-unit tiles.  The layer-by-layer form is
+reached by the same network with its inputs padded to 260 columns of zero
+weight: the same products in the same order, so equal bits; and against the
+oracle."""
+import numpy as np
+import pytest
+
+from oracle import mlp_ref as R
+from tests.helpers import dev, host
+from tests.test_mlp import BINGHAM_HEAD
+
+
+def _net(n_in, width, depth):
+    from cudimot_amd import capi
+    head = [capi.head_entry(e["kind"], e["param"], e["param2"], e["lo"], e["hi"], e["weight"], e["vmin"], e["vmax"])
+            for e in BINGHAM_HEAD]
+    return capi.Mlp(n_in, head, width=width, depth=depth, seed=3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,n_in,width,depth", [(1, 99, 256, 3), (32, 64, 128, 2), (33, 65, 32, 1), (63, 256, 96, 7),
+                                                (65, 1, 160, 2), (1000, 129, 256, 1), (70001, 99, 224, 3)])
+def test_one_launch_equals_layer_by_layer(n, n_in, width, depth):
+    import torch
+    from cudimot_amd import capi
+    net, wide = _net(n_in, width, depth), _net(260, width, depth)
+    w = net.get_weights()
+    first = np.zeros((width, 260), dtype=np.float32)
+    first[:, :n_in] = w[:width * n_in].reshape(width, n_in)
+    wide.set_weights(np.concatenate([first.ravel(), w[width * n_in:]]))
+    rng = np.random.default_rng(n)
+    x = rng.uniform(50.0, 1500.0, size=(n, n_in)).astype(np.float32)
+    xw = np.zeros((n, 260), dtype=np.float32)
+    xw[:, :n_in] = x
+    scale = rng.uniform(800.0, 1200.0, size=n).astype(np.float32)
+    res = []
+    for m, inp in ((net, x), (wide, xw)):
+        out, params = torch.empty((n, m.n_out), device="cuda"), dev(np.full((n, 7), 1.5))
+        m.forward(dev(inp), dev(scale), out)
+        m.init_params(dev(inp), dev(scale), params)
+        capi.sync()
+        res.append((host(out), host(params)))
+    np.testing.assert_array_equal(res[0][0], res[1][0])
+    np.testing.assert_array_equal(res[0][1], res[1][1])
+    ref, _ = R.forward(R.unflatten(w, net.layer_shapes()), x[-200:] / scale[-200:, None], bf16=True)
+    assert np.abs(res[0][0][-200:] - ref).max() / np.abs(ref).max() < 1e-2
