@@ -55,6 +55,13 @@ static size_t op_lds(const cdm::Geom& g) {
   return (size_t)cdm_mc_offset(g.nmeas, g.cfp_ts) * sizeof(float) + (size_t)g.nmeas * cdm_mc * sizeof(CDM_F64);
 }
 
+// Predicted signal and BIC/AIC: the voxels' mean samples share the space of the
+// tables staged after them.
+static size_t op_lds_post(const cdm::Geom& g, int L) {
+  const size_t means = (size_t)(cdm_block / L) * (cdm_np + 1) * sizeof(double), tables = op_lds(g);
+  return means > tables ? means : tables;
+}
+
 // LM launches: the 64-lane groups' J^T J scratch after the shared tables.
 static size_t op_lds_lm(const cdm::Geom& g, int L) {
   const size_t extra = cdm_lm_scratch_doubles(L, g.nmeas);

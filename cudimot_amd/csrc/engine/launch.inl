@@ -281,8 +281,8 @@ static hipError_t op_predicted(int L, const cdm::Geom& g, int nsamples, const fl
   a.tau_samples = nullptr;
   a.out = out;
   a.bic = a.aic = nullptr;
-  CDM_DISPATCH_L(L, hipLaunchKernelGGL(cdm_predicted_kernel<LG>, op_grid(g.nvox, LG), dim3(cdm_block), op_lds(g), s,
-                                       a));
+  CDM_DISPATCH_L(L, hipLaunchKernelGGL(cdm_predicted_kernel<LG>, op_grid(g.nvox, LG), dim3(cdm_block),
+                                       op_lds_post(g, LG), s, a));
   return hipGetLastError();
 }
 
@@ -300,10 +300,10 @@ static hipError_t op_bic_aic(int L, int rician, const cdm::Geom& g, int nsamples
   a.aic = aic;
   if (rician) {
     CDM_DISPATCH_L(L, hipLaunchKernelGGL((cdm_bic_aic_kernel<LG, true>), op_grid(g.nvox, LG), dim3(cdm_block),
-                                         op_lds(g), s, a));
+                                         op_lds_post(g, LG), s, a));
   } else {
     CDM_DISPATCH_L(L, hipLaunchKernelGGL((cdm_bic_aic_kernel<LG, false>), op_grid(g.nvox, LG), dim3(cdm_block),
-                                         op_lds(g), s, a));
+                                         op_lds_post(g, LG), s, a));
   }
   return hipGetLastError();
 }
