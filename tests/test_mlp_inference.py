@@ -46,3 +46,30 @@ def test_one_launch_equals_layer_by_layer(n, n_in, width, depth):
     np.testing.assert_array_equal(res[0][1], res[1][1])
     ref, _ = R.forward(R.unflatten(w, net.layer_shapes()), x[-200:] / scale[-200:, None], bf16=True)
     assert np.abs(res[0][0][-200:] - ref).max() / np.abs(ref).max() < 1e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_in,width,depth,batch", [(99, 256, 3, 2048), (64, 32, 1, 32), (256, 96, 7, 96),
+                                                    (33, 160, 2, 64)])
+def test_one_launch_training_step_follows_the_loss_gradient(n_in, width, depth, batch):
+    """One step (one batch, hardly any noise) against the loss and gradient of
+    the layer-by-layer launches at the same weights: Adam's first step is
+    -lr g / (|g| + 1e-8), so -lr sign(g) to 0.1% where |g| > 1e-5.  An input
+    that the residual noise moves over a BF16 rounding boundary (2^-9 of it)
+    can turn the sign of a gradient near zero only."""
+    from cudimot_amd import capi
+    from tests.test_mlp import bingham_truth
+    net = _net(n_in, width, depth)
+    rng = np.random.default_rng(batch)
+    x = rng.uniform(0.1, 1.5, size=(batch, n_in)).astype(np.float32)
+    t = dev(bingham_truth(batch, 4))
+    w0 = net.get_weights()
+    loss, g = net.loss_grad(dev(x), None, t)
+    lr = 1e-3
+    losses = net.train(dev(x), None, t, epochs=1, batch=batch, lr=lr, seed=1, snr=(1e9, 1e9))
+    step = (net.get_weights().astype(np.float64) - w0) / lr
+    assert abs(losses[0] - loss) <= 1e-4 * abs(loss), (losses, loss)
+    big = np.abs(g) > 1e-5
+    assert big.any()
+    close = np.abs(step[big] + np.sign(g[big])) < 2e-3 + 2.0 ** -22 * np.abs(w0[big]) / lr
+    assert close.mean() > 0.999, close.mean()
