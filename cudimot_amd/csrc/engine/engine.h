@@ -3109,7 +3109,8 @@ struct cdm_post_args {
 
 // The mean samples of the block's voxels, handed to each voxel's lanes in mp
 // (and the mean tau, with tau_samples): 16 lanes per row of samples, so that a
-// wave reads runs of adjacent values, into the dynamic LDS before anything else
+// wave reads runs of adjacent values (a thread per row below 16 samples, where
+// adjacent rows are near enough and 16 rows at a time are too few), into the dynamic LDS before anything else
 // is staged there.  Every lane of a voxel reading all of its samples by itself
 // took most of these kernels (NODDI_Bingham, 200k voxels, 50 samples, 99
 // measurements: predicted signal 0.48 -> 0.20 ms, BIC/AIC 0.54 -> 0.28 ms).
@@ -3122,15 +3123,27 @@ __device__ __forceinline__ void cdm_mean_samples(const cdm_post_args& a, double*
   const int v0 = blockIdx.x * per, nv = min(per, a.g.nvox - v0);
   const int lane = threadIdx.x % cdm_mean_lanes, S = a.nsamples;
   const int width = cdm_np + (rician ? 1 : 0);
-  for (int r = threadIdx.x / cdm_mean_lanes; r < nv * width; r += rows) {
-    const int q = r / width, i = r - q * width;
-    const float* s = i < cdm_np ? a.samples + ((size_t)(v0 + q) * cdm_np + i) * S
-                                : a.tau_samples + (size_t)(v0 + q) * S;
-    double acc = 0.0;
+  auto row = [&](int q, int i) {
+    return i < cdm_np ? a.samples + ((size_t)(v0 + q) * cdm_np + i) * S : a.tau_samples + (size_t)(v0 + q) * S;
+  };
+  if (S < cdm_mean_lanes) {
+    for (int r = threadIdx.x; r < nv * width; r += cdm_block) {
+      const int q = r / width, i = r - q * width;
+      const float* s = row(q, i);
+      double acc = 0.0;
+      for (int k = 0; k < S; ++k) acc += s[k];
+      s_mean[q * (cdm_np + 1) + i] = S > 1 ? acc / S : acc;
+    }
+  } else {
+    for (int r = threadIdx.x / cdm_mean_lanes; r < nv * width; r += rows) {
+      const int q = r / width, i = r - q * width;
+      const float* s = row(q, i);
+      double acc = 0.0;
 #pragma unroll 4
-    for (int k = lane; k < S; k += cdm_mean_lanes) acc += s[k];
-    acc = cdm::Group<cdm_mean_lanes>::sum(acc);
-    if (lane == 0) s_mean[q * (cdm_np + 1) + i] = S > 1 ? acc / S : acc;
+      for (int k = lane; k < S; k += cdm_mean_lanes) acc += s[k];
+      acc = cdm::Group<cdm_mean_lanes>::sum(acc);
+      if (lane == 0) s_mean[q * (cdm_np + 1) + i] = acc / S;
+    }
   }
   __syncthreads();
   const int q = threadIdx.x / L;
