@@ -67,12 +67,16 @@ PEAK_F32 = 157.3e12
 # and a 100-jump launch recording 10 samples), scaled by the same counters'
 # readings for a 512 MiB copy (fetch x2.0, write x1.0):
 # - per voxel and launch: the measurements read, the chain state and
-#   parameters written (burn-in launch: 55,904 + 36,380 KiB / 131,072 voxels);
-# - per stored sample value: one 32-byte sector, since a launch stores one
-#   sample of each parameter per recording and a parameter's samples lie
-#   contiguous per voxel ((30,214 + 250,002) KiB / 9,175,040 stores).
+#   parameters written (721 B);
+# - per voxel and jump: 32 bytes of scratch per lane that the steps in an angle
+#   write (burn-in launch: 309,283 + 3,003,687 KiB / 131,072 voxels, less the
+#   721 B, over 100 jumps);
+# - per stored sample value: one 32-byte sector and more, since a launch stores
+#   one sample of each parameter per recording and a parameter's samples lie
+#   contiguous per voxel ((30,659 + 331,689) KiB / 9,175,040 stores).
 MCMC_BYTES_PER_VOXEL_LAUNCH = 721.0
-MCMC_BYTES_PER_SAMPLE_STORE = 31.3
+MCMC_BYTES_PER_VOXEL_JUMP = 251.6
+MCMC_BYTES_PER_SAMPLE_STORE = 40.4
 SNR = 25.0
 S0 = 1000.0
 
@@ -498,11 +502,13 @@ def main():
                 "achieved": round(frac * PEAK_F64 / 1e12, 3), "peak": PEAK_F64 / 1e12, "unit": "TFLOP/s",
                 "frac": round(frac, 4),
                 "traffic": args.voxels * (2 * MCMC_BYTES_PER_VOXEL_LAUNCH +
+                                          (args.burnin + args.jumps) * MCMC_BYTES_PER_VOXEL_JUMP +
                                           P * nsamp * MCMC_BYTES_PER_SAMPLE_STORE) / 2,
                 "traffic_note": "HBM bytes per launch (mean of the burn-in and recording launches) from rocprofv3 "
                                 "FETCH_SIZE/WRITE_SIZE, copy-calibrated: measurements and chain state per voxel, "
-                                "one 32-byte sector per stored sample; the cache rows stay in LDS and nothing "
-                                "spills, so the kernel is bound by vector-ALU issue, not HBM",
+                                "32 bytes of scratch per lane written by the steps in an angle, a sector per "
+                                "stored sample; the cache rows stay in LDS: 0.1 TB/s, so the kernel is bound by "
+                                "vector-ALU issue, not HBM",
                 "flops_per_launch_f32": f32 / 2, "flops_per_launch_f64": f64 / 2,
                 "avg_launch_ms": mcmc_s * 1000 / 2,
                 "per_eval": {k: round(float(v), 2) for k, v in ev.items()}}
