@@ -42,6 +42,11 @@ struct GraphStats {
   long long captures = 0, replays = 0;
 };
 
+struct GsScratch {
+  void* p = nullptr;
+  size_t bytes = 0;
+};
+
 }  // namespace
 
 struct cdm_model {
@@ -73,10 +78,12 @@ struct cdm_model {
   size_t state_bytes = 0;
   // LM work-queue counter (one int; calls on one handle are serialised)
   int* d_queue = nullptr;
-  // scratch of a GridSearch split over slices of the combinations
-  // (cdm::gs_split_bytes), grown as needed
-  void* d_gs_split = nullptr;
-  size_t gs_split_bytes = 0;
+  // GridSearch scratch, grown as needed: of the scan split over slices of the
+  // combinations (cdm::gs_split_bytes), and of the search over basis signals
+  // (cdm::gs_work_bytes).  A caller's graph may hold the first: what it outgrew
+  // is kept until the handle is closed (at most its present size in all).
+  GsScratch gs_split, gs_basis;
+  std::vector<void*> gs_split_old;
   // MCMC phases recorded into HIP graphs (jump blocks with use_graph), one
   // per phase, and the private stream they are captured on
   GraphCache mcmc_graphs[2];
@@ -576,7 +583,9 @@ void cdm_model_close(cdm_model* m) {
   free_grid(m);
   if (m->d_state) (void)hipFree(m->d_state);
   if (m->d_queue) (void)hipFree(m->d_queue);
-  if (m->d_gs_split) (void)hipFree(m->d_gs_split);
+  for (GsScratch* b : {&m->gs_split, &m->gs_basis})
+    if (b->p) (void)hipFree(b->p);
+  for (void* p : m->gs_split_old) (void)hipFree(p);
   for (GraphCache& g : m->mcmc_graphs) g.clear();
   if (m->capture_stream) (void)hipStreamDestroy(m->capture_stream);
   if (m->last_done) (void)hipEventDestroy(m->last_done);
@@ -754,21 +763,31 @@ int gs_splits(int L, int nvox, int ncombs, int most) {
   return (int)std::max<long long>(1, S);
 }
 
-// The handle's GridSearch scratch, at least `bytes`, ordered after the
+// The handle's scratch of the split scan, at least `bytes`, ordered after the
 // handle's last call (its previous user).
-static hipError_t gs_scratch(cdm_model* m, size_t bytes, hipStream_t s) {
-  hipError_t e = order_after_last(m, s);
-  if (e != hipSuccess || m->gs_split_bytes >= bytes) return e;
-  if (m->has_last && (e = hipStreamSynchronize(m->last_stream)) != hipSuccess) return e;
-  if (m->d_gs_split) (void)hipFree(m->d_gs_split);
-  m->d_gs_split = nullptr;
-  m->gs_split_bytes = 0;
-  if ((e = hipMalloc(&m->d_gs_split, bytes)) != hipSuccess) {
-    m->d_gs_split = nullptr;
-    return e;
-  }
-  m->gs_split_bytes = bytes;
+static hipError_t gs_split_scratch(cdm_model* m, size_t bytes, hipStream_t s) {
+  const hipError_t e = order_after_last(m, s);
+  if (e != hipSuccess || m->gs_split.bytes >= bytes) return e;
+  bytes = std::max(bytes, 2 * m->gs_split.bytes);
+  void* p = nullptr;
+  const hipError_t ea = hipMalloc(&p, bytes);
+  if (ea != hipSuccess) return ea;
+  if (m->gs_split.p) m->gs_split_old.push_back(m->gs_split.p);
+  m->gs_split = {p, bytes};
   return hipSuccess;
+}
+
+// The same for the search over basis signals, which no graph holds.
+static hipError_t gs_basis_scratch(cdm_model* m, size_t bytes, hipStream_t s) {
+  hipError_t e = order_after_last(m, s);
+  GsScratch& b = m->gs_basis;
+  if (e != hipSuccess || b.bytes >= bytes) return e;
+  if (m->has_last && (e = hipStreamSynchronize(m->last_stream)) != hipSuccess) return e;
+  if (b.p) (void)hipFree(b.p);
+  b = {};
+  void* p = nullptr;
+  if ((e = hipMalloc(&p, bytes)) == hipSuccess) b = {p, bytes};
+  return e;
 }
 
 // Lanes per voxel of a search over basis signals: 4 (16 past 192
@@ -794,35 +813,45 @@ int cdm_gridsearch(cdm_model* m, int nvox, int nmeas, const float* meas, float* 
   const cdm::Consts c = make_consts(m);
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSuccess;
-  // The search over basis signals keeps its lists in the handle's scratch; a
-  // capturing caller gets the scan that needs none for a volume that fills
-  // the GPU.
+  // The search over basis signals keeps its lists in the handle's scratch,
+  // which a later call may replace; a capturing caller, whose graph would hold
+  // it, gets the scan.
   hipStreamCaptureStatus cst = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cst) != hipSuccess) {
     (void)hipGetLastError();
     cst = hipStreamCaptureStatusActive;
   }
-  const int LB = cst == hipStreamCaptureStatusNone ? gs_basis_lanes(m, g) : 0;
-  if (LB) {
-    const int S = std::min(m->plan.nshared, gs_splits(LB, nvox, INT_MAX, m->plan.nshared));
-    const int SB = std::max(1, std::min(m->plan.nshared, (4 << 20) / nvox));
-    if ((e = gs_scratch(m, cdm::gs_work_bytes(nvox, S, SB), s)) != hipSuccess)
-      return hip_fail(e, "GridSearch scratch");
-    if ((e = debug_reset(m, 0, s)) != hipSuccess) return hip_fail(e, "GridSearch --debug records");
-    e = m->ops->gridsearch_basis(LB, g, params, m->plan, c, kept,
-                                 cdm::gs_work_of(m->d_gs_split, nvox, S, SB, device_cus()), s);
-    if (e != hipSuccess) return hip_fail(e, "GridSearch launch");
-    (void)note_last(m, s);
-    return 0;
-  }
+  const bool capturing = cst != hipStreamCaptureStatusNone;
   const int L = group_for(m, cdm::kGridSearch, nmeas, nvox);
-  const int S = gs_splits(L, nvox, m->ncombs_valid, 16);
-  // the split search's lists belong to the handle too
-  if (S > 1 && (e = gs_scratch(m, cdm::gs_split_bytes(nvox, S), s)) != hipSuccess)
+  int S = gs_splits(L, nvox, m->ncombs_valid, 16);
+  const size_t split_bytes = S > 1 ? cdm::gs_split_bytes(nvox, S) : 0;
+  const int LB = capturing ? 0 : gs_basis_lanes(m, g);
+  if (LB) {
+    // the scan's scratch too, for the same call under capture: nothing can be
+    // allocated there
+    if (S > 1 && gs_split_scratch(m, split_bytes, s) != hipSuccess) (void)hipGetLastError();
+    const int SS = std::min(m->plan.nshared, gs_splits(LB, nvox, INT_MAX, m->plan.nshared));
+    const int SB = std::max(1, std::min(m->plan.nshared, (4 << 20) / nvox));
+    e = gs_basis_scratch(m, cdm::gs_work_bytes(nvox, SS, SB), s);
+    if (e == hipSuccess) {
+      if ((e = debug_reset(m, 0, s)) != hipSuccess) return hip_fail(e, "GridSearch --debug records");
+      e = m->ops->gridsearch_basis(LB, g, params, m->plan, c, kept,
+                                   cdm::gs_work_of(m->gs_basis.p, nvox, SS, SB, device_cus()), s);
+      if (e != hipSuccess) return hip_fail(e, "GridSearch launch");
+      (void)note_last(m, s);
+      return 0;
+    }
+    if (e != hipErrorOutOfMemory) return hip_fail(e, "GridSearch scratch");
+    (void)hipGetLastError();  // no memory for it: the scan
+  }
+  // the split scan's lists belong to the handle too; a capture without room for
+  // them scans in one slice
+  if (S > 1 && capturing && m->gs_split.bytes < split_bytes) S = 1;
+  if (S > 1 && (e = gs_split_scratch(m, split_bytes, s)) != hipSuccess)
     return hip_fail(e, "GridSearch scratch");
   if ((e = debug_reset(m, 0, s)) != hipSuccess) return hip_fail(e, "GridSearch --debug records");
   e = m->ops->gridsearch(L, g, params, (int)m->spec.grid_params.size(), m->spec.grid_params.data(), m->ncombs_valid,
-                         m->d_grid_f, m->d_grid_d, m->d_comb_id, c, kept, S, S > 1 ? m->d_gs_split : nullptr, s);
+                         m->d_grid_f, m->d_grid_d, m->d_comb_id, c, kept, S, S > 1 ? m->gs_split.p : nullptr, s);
   if (e != hipSuccess) return hip_fail(e, "GridSearch launch");
   if (S > 1) (void)note_last(m, s);
   return 0;
