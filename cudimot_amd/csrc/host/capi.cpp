@@ -11,7 +11,6 @@
 #include <cmath>
 #include <cstring>
 #include <fstream>
-#include <map>
 #include <mutex>
 #include <sstream>
 #include <string>
@@ -63,15 +62,15 @@ struct cdm_model {
   std::vector<Tuned> tuned;
   int mcmc_block = 0;
   int mcmc_graph = 0;
-  // device grid (valid combinations only)
+  // device grid (valid combinations only), and the grid ordered for the search
+  // over basis signals (plan.order null: the plug-in has no basis, or a value
+  // is listed twice); one allocation, d_grid
   bool grid_dirty = true;
   int ncombs_valid = 0;
+  void* d_grid = nullptr;
   float* d_grid_f = nullptr;
   double* d_grid_d = nullptr;
   int* d_comb_id = nullptr;
-  // the grid ordered for the search over basis signals (d_plan holds its
-  // tables; plan.order null: not a product, or the plug-in has no basis)
-  void* d_plan = nullptr;
   cdm::GridPlan plan = {};
   // MCMC chain state
   void* d_state = nullptr;
@@ -295,128 +294,108 @@ int check_geom(const cdm_model* m, int nvox, int nmeas, const void* meas, const 
 }
 
 void free_grid(cdm_model* m) {
-  if (m->d_grid_f) (void)hipFree(m->d_grid_f);
-  if (m->d_grid_d) (void)hipFree(m->d_grid_d);
-  if (m->d_comb_id) (void)hipFree(m->d_comb_id);
+  if (m->d_grid) (void)hipFree(m->d_grid);
+  m->d_grid = nullptr;
   m->d_grid_f = nullptr;
   m->d_grid_d = nullptr;
   m->d_comb_id = nullptr;
-  if (m->d_plan) (void)hipFree(m->d_plan);
-  m->d_plan = nullptr;
   m->plan = {};
 }
 
-// The grid's valid combinations (gf [n][ngp]) ordered by the plug-in's levels:
-// equal shared values together, within them equal values of every basis
-// parameter, each level in order of first appearance.  The search needs the
-// product structure a grid of per-parameter lists and per-parameter bounds
-// has; where it is not found the plan stays empty.
-int upload_plan(cdm_model* m, const std::vector<float>& gf, int n) {
-  const int ngp = (int)m->spec.grid_params.size();
-  if (!m->ops->grid_linear || n <= 0) return 0;
-  cdm::GridPlan p = {};
-  std::vector<int> cols[3];  // columns of the shared, the other basis and the weight parameters
-  for (int k = 0; k < ngp; ++k) {
-    const unsigned bit = 1u << m->spec.grid_params[k];
-    cols[(m->ops->grid_linear & bit) ? 2 : (m->ops->grid_shared & bit) ? 0 : 1].push_back(k);
-  }
-  // per level: each combination's index among the level's distinct tuples
-  std::vector<int> idx[3];
-  int count[3];
-  for (int l = 0; l < 3; ++l) {
-    std::map<std::vector<float>, int> seen;
-    idx[l].resize(n);
-    for (int c = 0; c < n; ++c) {
-      std::vector<float> key;
-      for (int k : cols[l]) key.push_back(gf[(size_t)c * ngp + k]);
-      idx[l][c] = seen.emplace(key, (int)seen.size()).first->second;
-    }
-    count[l] = (int)seen.size();
-  }
-  if ((long long)count[0] * count[1] * count[2] != n) return 0;
-  std::vector<int> order(n, -1);
-  for (int c = 0; c < n; ++c) {
-    const int at = (idx[0][c] * count[1] + idx[1][c]) * count[2] + idx[2][c];
-    if (order[at] >= 0) return 0;  // a repeated combination
-    order[at] = c;
-  }
-  const int np = m->ops->nparams;
-  std::vector<float> outer((size_t)count[0] * count[1] * np, 0.0f), inner((size_t)count[2] * np, 0.0f);
-  for (int o = 0; o < count[0] * count[1]; ++o)
-    for (int k = 0; k < ngp; ++k)
-      outer[(size_t)o * np + m->spec.grid_params[k]] = gf[(size_t)order[(size_t)o * count[2]] * ngp + k];
-  for (int j = 0; j < count[2]; ++j)
-    for (int k : cols[2]) inner[(size_t)j * np + m->spec.grid_params[k]] = gf[(size_t)order[j] * ngp + k];
-  const size_t nb = outer.size() * 4, ni = inner.size() * 4, no = order.size() * 4;
-  hipError_t e = hipMalloc(&m->d_plan, nb + ni + no);
-  if (e != hipSuccess) {
-    m->d_plan = nullptr;
-    return hip_fail(e, "grid");
-  }
-  char* d = (char*)m->d_plan;
-  if ((e = hipMemcpy(d, outer.data(), nb, hipMemcpyHostToDevice)) != hipSuccess ||
-      (e = hipMemcpy(d + nb, inner.data(), ni, hipMemcpyHostToDevice)) != hipSuccess ||
-      (e = hipMemcpy(d + nb + ni, order.data(), no, hipMemcpyHostToDevice)) != hipSuccess)
-    return hip_fail(e, "grid upload");
-  p.ngp = ngp;
-  p.ncombs = n;
-  p.gparams = m->spec.grid_params.data();
-  p.grid_f = m->d_grid_f;
-  p.grid_d = m->d_grid_d;
-  p.comb_id = m->d_comb_id;
-  p.nshared = count[0];
-  p.nouter = count[1];
-  p.ninner = count[2];
-  p.outer_vals = (const float*)d;
-  p.inner_vals = (const float*)(d + nb);
-  p.order = (const int*)(d + nb + ni);
-  m->plan = p;
-  return 0;
+// Whether the values from `first` on name one twice (as the floats that the
+// screen reads), or one that is not a number.
+bool has_repeats(const std::vector<double>& vals, size_t first) {
+  std::vector<float> v(vals.begin() + first, vals.end());
+  if (std::any_of(v.begin(), v.end(), [](float x) { return x != x; })) return true;
+  std::sort(v.begin(), v.end());
+  return std::adjacent_find(v.begin(), v.end()) != v.end();
 }
 
-// Combinations whose grid values pass the float bounds test of
-// GridSearch.cu:25-47; the non-grid parameters are tested per voxel on the
-// device.
+// The device grid: the product of each parameter's values that pass the float
+// bounds test of GridSearch.cu:25-47 (the non-grid parameters are tested per
+// voxel on the device), the lowest parameter outermost.  For plug-ins with
+// basis signals also the plan, the same combinations ordered by the plug-in's
+// levels: equal shared values together, within them equal values of every basis
+// parameter.  The host sends the lists and a kernel forms the product: a fit
+// loads its grid anew, so this counts in every first call (one voxel, 262,144
+// combinations of three parameters: 0.54 ms in all; with the product formed on
+// the host, and a map from values to their place in a level, 26 ms).
 int upload_grid(cdm_model* m) {
   if (!m->grid_dirty) return 0;
   free_grid(m);
   const cdm::ModelSpec& s = m->spec;
-  const int ngp = (int)s.grid_params.size();
-  std::vector<float> gf;
-  std::vector<double> gd;
-  std::vector<int> id;
-  for (int c = 0; c < s.grid_combs; ++c) {
-    bool ok = true;
-    for (int k = 0; k < ngp; ++k) {
-      const int p = s.grid_params[k];
-      const double v = s.grid[(size_t)c * ngp + k];
-      const float lo = (float)s.bmin[p], hi = (float)s.bmax[p];
-      const int bt = s.bound_types[p];
-      if ((bt == cdm::BMIN || bt == cdm::BMINMAX) && v < lo) ok = false;
-      if ((bt == cdm::BMAX || bt == cdm::BMINMAX) && v > hi) ok = false;
+  const int ngp = (int)s.grid_params.size(), np = m->ops->nparams;
+  cdm::GridFill f;
+  std::memset(&f, 0, sizeof(f));
+  std::vector<double> vals;  // every parameter's values inside its bounds
+  std::vector<int> ids;      // what each adds to the index among all combinations
+  size_t n = ngp > 0 ? 1 : 0, nl[3] = {1, 1, 1};
+  bool plan = m->ops->grid_linear != 0;
+  int stride = s.grid_combs;
+  for (int k = 0; k < ngp; ++k) {
+    const std::vector<double>& list = s.grid_vals[k];
+    const int p = s.grid_params[k], bt = s.bound_types[p];
+    const float lo = (float)s.bmin[p], hi = (float)s.bmax[p];
+    const int level = ((m->ops->grid_linear >> p) & 1u) ? 2 : ((m->ops->grid_shared >> p) & 1u) ? 0 : 1;
+    stride /= (int)list.size();
+    const size_t first = vals.size();
+    for (size_t i = 0; i < list.size(); ++i) {
+      const double v = list[i];
+      if ((bt == cdm::BMIN || bt == cdm::BMINMAX) && v < lo) continue;
+      if ((bt == cdm::BMAX || bt == cdm::BMINMAX) && v > hi) continue;
+      vals.push_back(v);
+      ids.push_back((int)i * stride);
     }
-    if (!ok) continue;
-    for (int k = 0; k < ngp; ++k) {
-      gd.push_back(s.grid[(size_t)c * ngp + k]);
-      gf.push_back((float)s.grid[(size_t)c * ngp + k]);
-    }
-    id.push_back(c);
+    f.axis[k] = {p, level, (int)first, (int)(vals.size() - first)};
+    n *= vals.size() - first;
+    nl[level] *= vals.size() - first;
+    plan = plan && !has_repeats(vals, first);
   }
-  m->ncombs_valid = (int)id.size();
-  if (m->ncombs_valid > 0) {
-    hipError_t e;
-    if ((e = hipMalloc((void**)&m->d_grid_f, gf.size() * sizeof(float))) != hipSuccess) return hip_fail(e, "grid");
-    if ((e = hipMalloc((void**)&m->d_grid_d, gd.size() * sizeof(double))) != hipSuccess) return hip_fail(e, "grid");
-    if ((e = hipMalloc((void**)&m->d_comb_id, id.size() * sizeof(int))) != hipSuccess) return hip_fail(e, "grid");
-    if ((e = hipMemcpy(m->d_grid_f, gf.data(), gf.size() * sizeof(float), hipMemcpyHostToDevice)) != hipSuccess)
-      return hip_fail(e, "grid upload");
-    if ((e = hipMemcpy(m->d_grid_d, gd.data(), gd.size() * sizeof(double), hipMemcpyHostToDevice)) != hipSuccess)
-      return hip_fail(e, "grid upload");
-    if ((e = hipMemcpy(m->d_comb_id, id.data(), id.size() * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess)
-      return hip_fail(e, "grid upload");
-    const int r = upload_plan(m, gf, m->ncombs_valid);
-    if (r) return r;
+  m->ncombs_valid = (int)n;
+  if (n == 0) {
+    m->grid_dirty = false;
+    return 0;
   }
+  // one buffer: the lists (doubles, then ints), [n][ngp] values, the indices, the plan's tables
+  const size_t nv = vals.size(), lists = nv * 8 + (nv + 1) / 2 * 8, grid = n * ((size_t)ngp * 12 + 4);
+  hipError_t e = hipErrorOutOfMemory;
+  if (plan) e = hipMalloc(&m->d_grid, lists + grid + (nl[0] * nl[1] + nl[2]) * np * 4 + n * 4);
+  if (e != hipSuccess) {  // no plan, or no memory for its tables
+    (void)hipGetLastError();
+    plan = false;
+    e = hipMalloc(&m->d_grid, lists + grid);
+  }
+  if (e != hipSuccess) {
+    m->d_grid = nullptr;
+    return hip_fail(e, "grid");
+  }
+  std::vector<char> up(lists);
+  std::memcpy(up.data(), vals.data(), nv * 8);
+  std::memcpy(up.data() + nv * 8, ids.data(), nv * 4);
+  char* d = (char*)m->d_grid;
+  f.n = (int)n;
+  f.ngp = ngp;
+  f.nparams = np;
+  f.vals = (const double*)d;
+  f.ids = (const int*)(d + nv * 8);
+  f.grid_d = (double*)(d + lists);
+  f.grid_f = (float*)(f.grid_d + n * ngp);
+  f.comb_id = (int*)(f.grid_f + n * ngp);
+  if (plan) {
+    for (int l = 0; l < 3; ++l) f.levels[l] = (int)nl[l];
+    f.outer = (float*)(f.comb_id + n);
+    f.inner = f.outer + nl[0] * nl[1] * np;
+    f.order = (int*)(f.inner + nl[2] * np);
+  }
+  if ((e = hipMemcpy(d, up.data(), lists, hipMemcpyHostToDevice)) != hipSuccess ||
+      (e = cdm::grid_fill(f, nullptr)) != hipSuccess || (e = hipStreamSynchronize(nullptr)) != hipSuccess)
+    return hip_fail(e, "grid upload");
+  m->d_grid_f = f.grid_f;
+  m->d_grid_d = f.grid_d;
+  m->d_comb_id = f.comb_id;
+  if (plan)
+    m->plan = {ngp, (int)n, s.grid_params.data(), f.grid_f, f.grid_d, f.comb_id, f.levels[0], f.levels[1], f.levels[2],
+               f.outer, f.inner, f.order};
   m->grid_dirty = false;
   return 0;
 }

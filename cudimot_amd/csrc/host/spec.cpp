@@ -202,11 +202,13 @@ std::string parse_grid_text(const std::string& text, ModelSpec& spec) {
     }
   }
   spec.grid_params.clear();
+  spec.grid_vals.clear();
   spec.grid.clear();
   spec.grid_combs = 1;
   for (int i = 0; i < spec.nparams; ++i)
     if (!vals[i].empty()) {
       spec.grid_params.push_back(i);
+      spec.grid_vals.push_back(vals[i]);
       spec.grid_combs *= (int)vals[i].size();
     }
   if (spec.grid_params.empty()) {

@@ -31,6 +31,7 @@ struct ModelSpec {
 
   // Grid search
   std::vector<int> grid_params;  // ascending parameter ids
+  std::vector<std::vector<double>> grid_vals;  // each one's values, as listed
   int grid_combs = 0;
   std::vector<double> grid;      // [grid_combs][grid_params.size()]
 };
