@@ -902,7 +902,7 @@ static_assert((cdm_gs_shared & cdm_gs_linear) == 0 && (cdm_gs_table_dep & ~cdm_g
 #else
 constexpr bool cdm_gs_basis = false;
 constexpr unsigned cdm_gs_linear = 0, cdm_gs_shared = 0, cdm_gs_table_dep = 0, cdm_gs_frame_dep = 0;
-constexpr int cdm_gs_ntab = 0, cdm_gs_ns = 1, cdm_gs_nc = 0, cdm_gs_nw = 0;
+constexpr int cdm_gs_ntab = 0, cdm_gs_ns = 1, cdm_gs_ks = 0, cdm_gs_nc = 0, cdm_gs_nw = 0;
 #endif
 constexpr int cdm_gs_row = cdm_gs_ns + 1;  // values per measurement of a voxel's LDS rows: Grid_Shared's, the measurement
 

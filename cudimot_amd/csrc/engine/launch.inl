@@ -105,13 +105,41 @@ static cdm_gs_plan op_gs_plan(int L, const cdm::Geom& g, const cdm::GridPlan& p,
   return k;
 }
 
-static int op_grid_basis_lanes(int L, const cdm::Geom& g, const cdm::GridPlan& p) {
+// Whether the scan of every combination is the better search: a grid that moves
+// no weight, where an evaluation of the basis serves one combination.  Ratios
+// are this search's time to the scan's, at 20k voxels unless said; slots: the
+// lanes that fill the GPU.
+// - A single combination: 26 and 21 us.
+// - Sticks, each combination with its own shared part, several shared signals
+//   (directions of the first stick): Ball_3_Sticks 0.8 at 30 measurements, 1.1 at 45,
+//   1.8 at 90, 2.6 at 280, 150k voxels 1.8 to 2.9; small volumes gain by the slices
+//   of the shared combinations (3,000 voxels 0.5 at 30, 1.0 at 90, 1.7 at 280).
+// - The same with the ball alone shared (Ball_1_Stick, diffusivities): 1.0 up to 64
+//   measurements, 1.2 to 2.3 from 90 on; 150k voxels 0.6 to 1.0.
+// - Sticks, several combinations to a shared part.  The ball alone: directions 1.3
+//   to 1.7, with diffusivities 0.8 to 1.6, 150k voxels 0.7 to 1.1, 604 measurements
+//   1.2.  Several shared signals: 0.5 to 0.9, but 1.1 to 1.3 at 3,000 voxels with a
+//   single shared part, which has no slices.
+static bool op_gs_scan_better(const cdm::Geom& g, const cdm::GridPlan& p, long long slots) {
+  if (p.ncombs < 2) return true;
+  if (p.ninner > 1 || cdm_gs_ntab > 0) return false;
+  const bool idle = (long long)g.nvox * 16 < slots, large = (long long)g.nvox * 16 >= 10 * slots;
+  if (cdm_gs_ks > 1)
+    return p.nouter > 1 ? p.nshared == 1 && idle : (long long)g.nvox * g.nmeas >= (g.nmeas < 40 ? 5 : 2) * slots;
+  return p.nouter > 1 ? !large || g.nmeas >= 480 : !large && g.nmeas >= 80;
+}
+
+// Lanes the search over basis signals runs at, from L on those whose LDS fits;
+// 0: the scan is taken, also where no weight moves and even 64 lanes leave one
+// block per CU (NODDI_Watson, 604 measurements, 432 combinations, 20k voxels: 70
+// ms against 46).
+static int op_grid_basis_lanes(int L, const cdm::Geom& g, const cdm::GridPlan& p, long long slots) {
   if constexpr (!cdm_gs_basis) return 0;
-  if ((size_t)p.ninner * cdm_gs_nw * sizeof(float) > cdm_gs_table_max) return 0;
+  if ((size_t)p.ninner * cdm_gs_nw * sizeof(float) > cdm_gs_table_max || op_gs_scan_better(g, p, slots)) return 0;
   for (; L <= 64; L *= 4) {
     size_t lds = 0;
     (void)op_gs_plan(L, g, p, &lds);
-    if (lds <= cdm_lds_max) return L;
+    if (lds <= cdm_lds_max) return p.ninner == 1 && L == 64 && lds > cdm_lds_max / 2 ? 0 : L;
   }
   return 0;
 }

@@ -778,7 +778,7 @@ static int gs_basis_lanes(const cdm_model* m, const cdm::Geom& g) {
   int L = m->group[cdm::kGridSearch];
   if (!L)
     for (L = g.nmeas >= 192 ? 16 : 4; L < 64 && (long long)g.nvox * L * m->plan.nshared < kLaneSlots;) L *= 4;
-  return m->ops->grid_basis_lanes(L, g, m->plan);
+  return m->ops->grid_basis_lanes(L, g, m->plan, kLaneSlots);
 }
 
 int cdm_gridsearch(cdm_model* m, int nvox, int nmeas, const float* meas, float* params, const float* cfp,

@@ -145,9 +145,10 @@ struct ModelOps {
   int (*mcmc_rows_lds)(int L, int W, const Geom& g);
   // GridSearch over basis signals (plug-ins that declare CDM_GRID_LINEAR;
   // grid_linear 0: not available): the parameters of its levels, the lanes a
-  // search of this shape runs at (0: its LDS does not fit), and the search
+  // search of this shape runs at (0: the scan is taken; slots: the lanes that fill
+  // the GPU), and the search
   unsigned grid_linear, grid_shared;
-  int (*grid_basis_lanes)(int L, const Geom& g, const GridPlan& p);
+  int (*grid_basis_lanes)(int L, const Geom& g, const GridPlan& p, long long slots);
   hipError_t (*gridsearch_basis)(int L, const Geom& g, float* params, const GridPlan& p, const Consts& c, int* kept,
                                  const GridWork& w, hipStream_t s);
 };
