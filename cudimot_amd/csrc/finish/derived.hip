@@ -10,7 +10,12 @@
 // bound, 16 lanes per row of samples, so that a wave reads runs of adjacent
 // values (one thread per row had every lane of a wave on another row: 1.02 ms
 // for the 280 MB of 200k voxels x 7 x 50, against 0.105 ms; dyads 0.36-0.58 ->
-// 0.06-0.08 ms, maps 0.37 -> 0.035 ms).
+// 0.06-0.08 ms, maps 0.37 -> 0.035 ms).  Rows of few samples lie near enough for
+// a thread each, and 16 lanes would mostly idle: a million voxels, means of 1 / 4 /
+// 12 / 15 / 16 samples 25 / 46 / 157 / 219 / 272 us by threads and 196 / 199 / 244 /
+// 248 / 257 by 16 lanes; dyads of 1 / 4 / 8 / 12 samples 53 / 99 / 166 / 256 and 110 /
+// 166 / 167 / 179; Bingham maps of 4 / 8 samples 43 / 136 and 100 / 100, Watson's (one
+// row a voxel) of 2 / 4 23 / 64 and 50 / 51.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,19 +31,20 @@ namespace {
 constexpr int kBlock = 256;
 constexpr float kTwoDivPi = 0.636619772367581f;  // the finish scripts' Two_div_pi
 
-constexpr int kLanes = 16;  // lanes per row of samples
-constexpr int kPer = kBlock / kLanes;
-typedef cdm::Group<kLanes> Row;
+constexpr int kLanes = 16;  // lanes per row of samples, from kFew* samples on (one below)
+constexpr int kFewMean = 16, kFewDyads = 8, kFewBingham = 8, kFewWatson = 4;
 
+template <int LANES>
 __global__ __launch_bounds__(kBlock) void sample_mean_kernel(long long rows, int ns, const float* __restrict__ x,
                                                              float* __restrict__ out) {
-  const int lane = threadIdx.x % kLanes;
-  for (long long r = (long long)blockIdx.x * kPer + threadIdx.x / kLanes; r < rows; r += (long long)gridDim.x * kPer) {
+  constexpr int kPer = kBlock / LANES;
+  const int lane = threadIdx.x % LANES;
+  for (long long r = (long long)blockIdx.x * kPer + threadIdx.x / LANES; r < rows; r += (long long)gridDim.x * kPer) {
     const float* p = x + r * ns;
     double s = 0.0;
 #pragma unroll 4
-    for (int k = lane; k < ns; k += kLanes) s += p[k];
-    s = Row::sum(s);
+    for (int k = lane; k < ns; k += LANES) s += p[k];
+    s = cdm::Group<LANES>::sum(s);
     if (lane == 0) out[r] = (float)(s / ns);
   }
 }
@@ -79,28 +85,31 @@ __device__ void jacobi3(double a[3][3], double v[3][3]) {
   }
 }
 
-// A block handles kDyadVoxels voxels: the dyadic sums, 16 lanes per voxel, into
-// LDS, then one thread per voxel for the eigenvectors (a thousand serial FP64
-// instructions that 16 lanes would repeat).
-constexpr int kDyadVoxels = 64;
+// A block handles 64 voxels (a thread per row: 256): the dyadic sums, 16 lanes per
+// voxel, into LDS, then one thread per voxel for the eigenvectors (a thousand
+// serial FP64 instructions that 16 lanes would repeat).
+template <int LANES>
+constexpr int kDyadVoxels = LANES == 1 ? kBlock : 64;
 
 // Blocks of a launch over `n` units, `per` a block: at most kMaxBlocks (a launch
 // has fewer than 2^32 threads), which then take several each.
 constexpr long long kMaxBlocks = 1 << 20;
 unsigned blocks_for(long long n, int per) { return (unsigned)std::min((n + per - 1) / per, kMaxBlocks); }
 
+template <int LANES>
 __global__ __launch_bounds__(kBlock) void dyads_kernel(int n, int np, int ns, const float* __restrict__ x, int th,
                                                        int ph, int psi, float* __restrict__ dyads,
                                                        float* __restrict__ disp) {
-  __shared__ double sums[kDyadVoxels][7];  // 7: an odd stride over the banks
-  const int lane = threadIdx.x % kLanes;
-  for (long long v0 = (long long)blockIdx.x * kDyadVoxels; v0 < n; v0 += (long long)gridDim.x * kDyadVoxels) {
-    for (int q = threadIdx.x / kLanes; q < kDyadVoxels; q += kPer) {
+  constexpr int kVoxels = kDyadVoxels<LANES>, kPer = kBlock / LANES;
+  __shared__ double sums[kVoxels][7];  // 7: an odd stride over the banks
+  const int lane = threadIdx.x % LANES;
+  for (long long v0 = (long long)blockIdx.x * kVoxels; v0 < n; v0 += (long long)gridDim.x * kVoxels) {
+    for (int q = threadIdx.x / LANES; q < kVoxels; q += kPer) {
       const long long v = v0 + q;
       if (v >= n) break;
       const float* base = x + (size_t)v * np * ns;
       double m[6] = {};
-      for (int k = lane; k < ns; k += kLanes) {
+      for (int k = lane; k < ns; k += LANES) {
         const float t = base[th * ns + k], f = base[ph * ns + k];
         float st, ct, sf, cf;
         sincosf(t, &st, &ct);
@@ -125,13 +134,13 @@ __global__ __launch_bounds__(kBlock) void dyads_kernel(int n, int np, int ns, co
       }
 #pragma unroll
       for (int e = 0; e < 6; ++e) {
-        const double t = Row::sum(m[e]);
+        const double t = cdm::Group<LANES>::sum(m[e]);
         if (lane == 0) sums[q][e] = t;
       }
     }
     __syncthreads();
     const long long v = v0 + threadIdx.x;
-    if (threadIdx.x < kDyadVoxels && v < n) {
+    if (threadIdx.x < kVoxels && v < n) {
       double m[3][3];
       for (int i = 0, e = 0; i < 3; ++i)
         for (int j = i; j < 3; ++j, ++e) m[j][i] = m[i][j] = sums[threadIdx.x][e] / ns;
@@ -157,14 +166,16 @@ __global__ __launch_bounds__(kBlock) void dyads_kernel(int n, int np, int ns, co
   }
 }
 
+template <int LANES>
 __global__ __launch_bounds__(kBlock) void noddi_maps_kernel(int n, int np, int ns, const float* __restrict__ x,
                                                             int kappa, int beta, float* __restrict__ maps) {
-  const int lane = threadIdx.x % kLanes;
-  for (long long v = (long long)blockIdx.x * kPer + threadIdx.x / kLanes; v < n; v += (long long)gridDim.x * kPer) {
+  constexpr int kPer = kBlock / LANES;
+  const int lane = threadIdx.x % LANES;
+  for (long long v = (long long)blockIdx.x * kPer + threadIdx.x / LANES; v < n; v += (long long)gridDim.x * kPer) {
     const float* base = x + (size_t)v * np * ns;
     double sk = 0.0, sb = 0.0, sk2 = 0.0;
 #pragma unroll 4
-    for (int k = lane; k < ns; k += kLanes) {
+    for (int k = lane; k < ns; k += LANES) {
       const float kk = base[kappa * ns + k];
       sk += kk;
       if (beta >= 0) {
@@ -173,10 +184,10 @@ __global__ __launch_bounds__(kBlock) void noddi_maps_kernel(int n, int np, int n
         sk2 += (float)(kk - bb);  // the k2 = kappa - beta sample volume
       }
     }
-    sk = Row::sum(sk);
+    sk = cdm::Group<LANES>::sum(sk);
     if (beta >= 0) {
-      sb = Row::sum(sb);
-      sk2 = Row::sum(sk2);
+      sb = cdm::Group<LANES>::sum(sb);
+      sk2 = cdm::Group<LANES>::sum(sk2);
     }
     if (lane != 0) continue;
     const float mk = (float)(sk / ns);
@@ -209,8 +220,10 @@ int cdm_sample_mean(int nvox, int nparams, int nsamples, const float* samples, f
   if (nvox == 0) return 0;
   if (!samples || !mean) return cdm::set_error("cdm_sample_mean: null pointer");
   const long long rows = (long long)nvox * nparams;
-  hipLaunchKernelGGL(sample_mean_kernel, dim3(blocks_for(rows, kPer)), dim3(kBlock), 0,
-                     (hipStream_t)stream, rows, nsamples, samples, mean);
+  const bool few = nsamples < kFewMean;
+  hipLaunchKernelGGL(few ? sample_mean_kernel<1> : sample_mean_kernel<kLanes>,
+                     dim3(blocks_for(rows, few ? kBlock : kBlock / kLanes)), dim3(kBlock), 0, (hipStream_t)stream, rows,
+                     nsamples, samples, mean);
   return launch_check("cdm_sample_mean");
 }
 
@@ -221,8 +234,10 @@ int cdm_dyads(int nvox, int nparams, int nsamples, const float* samples, int the
     return cdm::set_error("cdm_dyads: parameter index out of range");
   if (nvox == 0) return 0;
   if (!samples || !dyads) return cdm::set_error("cdm_dyads: null pointer");
-  hipLaunchKernelGGL(dyads_kernel, dim3(blocks_for(nvox, kDyadVoxels)), dim3(kBlock), 0, (hipStream_t)stream, nvox,
-                     nparams, nsamples, samples, theta, phi, psi, dyads, dispersion);
+  const bool few = nsamples < kFewDyads;
+  hipLaunchKernelGGL(few ? dyads_kernel<1> : dyads_kernel<kLanes>,
+                     dim3(blocks_for(nvox, few ? kDyadVoxels<1> : kDyadVoxels<kLanes>)), dim3(kBlock), 0,
+                     (hipStream_t)stream, nvox, nparams, nsamples, samples, theta, phi, psi, dyads, dispersion);
   return launch_check("cdm_dyads");
 }
 
@@ -232,7 +247,9 @@ int cdm_noddi_maps(int nvox, int nparams, int nsamples, const float* samples, in
   if (kappa < 0 || kappa >= nparams || beta >= nparams) return cdm::set_error("cdm_noddi_maps: parameter index out of range");
   if (nvox == 0) return 0;
   if (!samples || !maps) return cdm::set_error("cdm_noddi_maps: null pointer");
-  hipLaunchKernelGGL(noddi_maps_kernel, dim3(blocks_for(nvox, kPer)), dim3(kBlock), 0, (hipStream_t)stream, nvox,
+  const bool few = nsamples < (beta >= 0 ? kFewBingham : kFewWatson);
+  hipLaunchKernelGGL(few ? noddi_maps_kernel<1> : noddi_maps_kernel<kLanes>,
+                     dim3(blocks_for(nvox, few ? kBlock : kBlock / kLanes)), dim3(kBlock), 0, (hipStream_t)stream, nvox,
                      nparams, nsamples, samples, kappa, beta, maps);
   return launch_check("cdm_noddi_maps");
 }
