@@ -552,7 +552,12 @@ __global__ void __launch_bounds__(64 * kInferWaves, 4)
 // Products, their order and the roundings are the layer-by-layer form's.
 // Measured, batch 2,048, 99 inputs, three layers of 256: seven launches, 56 us of
 // a step's 86, -> one of 31 us, step 61 us (batch 512: 75 -> 51).
+//   Past four blocks per CU a step waits for the matrix cores' idle rows instead:
+// layer by layer and in one launch, batch 4,096 105 and 92 us a step, 8,192 143
+// and 146 (layers of 128: 100 and 87), 16,384 218 and 250, 65,536 751 and 915;
+// layers of 32, 65,536: 202 and 311.  Larger batches go layer by layer.
 constexpr int kTrainRows = 8;
+constexpr int kTrainBatch = 8192;
 
 struct TrainNet {
   InferNet f;
@@ -1146,8 +1151,8 @@ TrainNet train_net(const cdm_mlp* m) {
   return t;
 }
 
-// Inference over n voxels in chunks: raw outputs to out [n][npad] (device,
-// caller's) or straight into the decode step.
+// Inference over n voxels, in one launch or layer by layer in chunks: raw outputs
+// to out_raw [n][n_out] and decoded parameters to params (either may be null).
 int infer(cdm_mlp* m, int n, int nmeas, const float* meas, const float* scale, float* out_raw, int nparams,
           float* params, hipStream_t s) {
   if (fits_one_launch(m)) {
@@ -1446,7 +1451,7 @@ int cdm_mlp_train(cdm_mlp* m, int n, int nmeas, const float* clean, const float*
     const float* tgt = tab ? target : target + (size_t)a.first * m->n_out;
     const float grad_scale = 1.0f / batch, loss_scale = 1.0f / (batch * (float)nb);
     const AdamStep st = adam_step_args(m, a.lr, tab, ctr);
-    if (fits_one_launch(m)) {
+    if (fits_one_launch(m) && batch <= kTrainBatch) {
       hipLaunchKernelGGL(train_rows_kernel, dim3(batch / kTrainRows), dim3(64 * kInferWaves),
                          (size_t)m->depth * kTrainRows * kInferK * sizeof(float), q, train_net(m), m->head, batch, tgt,
                          grad_scale, loss_scale, m->loss_sum, tab, ctr);
