@@ -2512,15 +2512,6 @@ __device__ __forceinline__ double cdm_neg_loglik(const cdm_geom& g, const float*
   for (int i = 0; i < cdm_np; ++i) pf[i] = (cdm_tf)p[i];
   cdm_cfp_row<cdm_tf> row;
   double acc = 0.0;
-  // The measurements come from memory (a wave's voxels outgrow the L1 cache),
-  // so a block of them is loaded ahead of the signals of the block before
-  // (Ball_2_Sticks MCMC, 280 measurements, 200k voxels: 3.64 -> 1.99 ns per voxel
-  // and jump at 4 lanes).
-  constexpr int U = RICIAN ? 1 : 4;
-  const int last = g.nmeas - 1;
-  float yb[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) yb[u] = mv[min(lane + u * L, last)];
   auto add = [&](int m, float ym) {
     const cdm_tf s = cdm_signal_f(pf, row.at(s_cfp, m, g.cfp_ts), fx, vc, cdm_mc_row(s_mc, m), fr);
     if constexpr (RICIAN) {
@@ -2532,18 +2523,42 @@ __device__ __forceinline__ double cdm_neg_loglik(const cdm_geom& g, const float*
     }
   };
   int m = lane;
-  for (; m + (U - 1) * L < g.nmeas; m += U * L) {
-    float yn[U];
+  if constexpr (RICIAN) {
+    for (; m < g.nmeas; m += L) add(m, mv[m]);
+  } else {
+    // The measurements come from memory (a wave's voxels outgrow the L1 cache),
+    // so a block of them is loaded ahead of the signals of the block before
+    // (Ball_2_Sticks MCMC, 280 measurements, 30k voxels, 96 jumps at 4 lanes: 14.2 ->
+    // 6.7 ms).  Whole blocks, counted for the group: their loads need no bound
+    // (with one for every load 7.4 ms, and light signals of few measurements, 64 of
+    // DiffusionTensor over 140k voxels, slower than without: 6.6 -> 7.4, now 6.9), and the
+    // last is loaded twice.  The Rician sum loads as it goes: its logarithms hide
+    // that (one load ahead: DiffusionTensor 26k voxels 4.8 -> 5.1 ms).
+    constexpr int U = 4;
+    const int last = g.nmeas - 1, blocks = g.nmeas / (U * L);
+    float y0 = mv[min(m + blocks * U * L, last)];  // the first of the rest
+    if (blocks > 0) {
+      const float* y = mv + m;
+      float yb[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) yn[u] = mv[min(m + (U + u) * L, last)];
+      for (int u = 0; u < U; ++u) yb[u] = y[u * L];
+      for (int k = 1; k <= blocks; ++k, m += U * L) {
+        y += k < blocks ? U * L : 0;
+        float yn[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) add(m + u * L, yb[u]);
+        for (int u = 0; u < U; ++u) yn[u] = y[u * L];
 #pragma unroll
-    for (int u = 0; u < U; ++u) yb[u] = yn[u];
+        for (int u = 0; u < U; ++u) add(m + u * L, yb[u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) yb[u] = yn[u];
+      }
+    }
+    for (; m < g.nmeas; m += L) {
+      const float ym = y0;
+      y0 = mv[min(m + L, last)];
+      add(m, ym);
+    }
   }
-#pragma unroll
-  for (int u = 0; u < U - 1; ++u)
-    if (m + u * L < g.nmeas) add(m + u * L, yb[u]);
   acc = cdm::Group<L>::sum(acc);
   if constexpr (RICIAN) return -g.nmeas * log(tau) - acc;
   else return (g.nmeas / 2.0) * log(acc / 2.0);
