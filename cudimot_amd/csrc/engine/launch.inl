@@ -246,11 +246,38 @@ static hipError_t op_levmar(int L, int W, const cdm::Geom& g, float* params, int
   return hipGetLastError();
 }
 
-// One MCMC launch: in time slices (cdm_mcmc_kernel) when the tiles outnumber the
-// resident blocks R without filling sixteen rounds of them, so that the last
-// round is at most a sixteenth of the launch; at least 16 jumps a slice, since
-// each slice rebuilds the voxel caches and cache rows (about 0.3 jumps).
+// Slices of an MCMC launch of `tiles` blocks, per_cu of them resident on each of
+// ncu compute units (cdm_mcmc_kernel).  Without slices the last round is as long
+// as a full one where two blocks per CU wait for their own results, and 0.4 of that
+// where more share the CU (they speed up as others leave); n slices take between
+// r = tiles / resident and ceil(n r) / n rounds, and each a hand-over (the chain
+// state through memory, an L2 write-back, the prologue) worth 250 likelihood terms of
+// a lane.  A step has ceil(M / L) terms, eight times the cost for plug-ins with a
+// voxel cache, and draws worth three.  At most as many slices as fill sixteen rounds, of
+// 16 jumps at least.  Measured with and without: NODDI_Bingham, 35k voxels (r = 1.07), 300
+// jumps 28.1 and 43.8 ms, 14k (1.7) 18.7 and 21.4; Ball_1_Stick, 66k (1.01), 300 jumps
+// 8.7 and 11.1, but 300k (4.6), 64 jumps 8.6 and 7.3; toymodel, 66k, 300 jumps 3.1 and
+// 2.6; DiffusionTensor, 300k, 64 jumps 9.8 and 9.0.
 constexpr int cdm_mcmc_rounds = 16, cdm_mcmc_least_jumps = 16;
+static int op_mcmc_slices(int tiles, int per_cu, int ncu, int count, int nmeas, int L) {
+  const long long R = (long long)per_cu * ncu;
+  if (R <= 0 || tiles <= R) return 1;
+  const long long want = (cdm_mcmc_rounds * R + tiles - 1) / tiles;
+  const int most = (int)std::min<long long>(want, count / cdm_mcmc_least_jumps);
+  const double r = (double)tiles / R, whole = (double)((tiles + R - 1) / R);
+  const double terms = (double)count * cdm_np * ((nmeas + L - 1) / L * (cdm_vc > 1 ? 8 : 1) + 3);
+  int n = 1;
+  double best = per_cu > 2 ? r + 0.4 * (whole - r) : whole;
+  for (int k = 2; k <= most; ++k) {
+    const double last = (double)(((long long)k * tiles + R - 1) / R) / k;
+    const double t = 0.5 * (r + last) * (1.0 + 250.0 * k / terms);
+    if (t < best) {
+      best = t;
+      n = k;
+    }
+  }
+  return n;
+}
 
 template <int L, bool RICIAN, int W>
 static hipError_t op_mcmc_launch(cdm_mcmc_args a, size_t lds, int* queue, int ncu, hipStream_t s) {
@@ -260,10 +287,8 @@ static hipError_t op_mcmc_launch(cdm_mcmc_args a, size_t lds, int* queue, int nc
     const hipError_t e =
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (cdm_mcmc_kernel<L, RICIAN, W>), cdm_block, lds);
     if (e != hipSuccess) return e;
-    const long long resident = (long long)per_cu * ncu;
-    const long long want = (cdm_mcmc_rounds * resident + a.ntiles - 1) / a.ntiles;
-    const int n = (int)std::min<long long>(want, a.count / cdm_mcmc_least_jumps);
-    if (resident > 0 && a.ntiles > resident && n > 1) {
+    const int n = op_mcmc_slices(a.ntiles, per_cu, ncu, a.count, a.g.nmeas, L);
+    if (n > 1) {
       a.queue = queue;
       a.chunk_len = (a.count + n - 1) / n;
       const unsigned slices = (unsigned)((a.count + a.chunk_len - 1) / a.chunk_len);
