@@ -885,17 +885,28 @@ int check_mcmc(cdm_model* m, int nvox, int nmeas, const float* meas, const float
   return 0;
 }
 
-// Register budget an MCMC launch runs at (the Rician likelihood is compiled
-// at the default budget only); with the voxel group it decides where the
-// per-measurement cache rows live.
-int mcmc_budget(const cdm_model* m, int nmeas, int rician) { return rician ? 1 : occ_for(m, cdm::kMcmc, nmeas); }
+// Register budget an MCMC launch of group size L runs at (the Rician likelihood
+// is compiled at the default budget only); with the voxel group it decides where
+// the per-measurement cache rows live.  A tuned budget is that of a volume that
+// fills the GPU: fewer blocks take the smallest budget that keeps all of them
+// resident, since more registers a wave cost nothing there (NODDI_Watson, tuned to
+// 4 blocks per CU, 300 voxels, 96 jumps at 4 and 1 blocks: 2.13 and 1.56 ms;
+// DiffusionTensor, 32k voxels at 4 and 2: 2.05 and 1.85).  An explicit one stands.
+int mcmc_budget(const cdm_model* m, int nmeas, int rician, int nvox, int L) {
+  if (rician) return 1;
+  int W = occ_for(m, cdm::kMcmc, nmeas);
+  if (m->occ[cdm::kMcmc]) return W;
+  const long long blocks = ((long long)nvox * L + 255) / 256, ncu = device_cus();
+  while (W > 1 && blocks <= W / 2 * ncu) W /= 2;
+  return W;
+}
 
 // Bytes of chain state an MCMC call over nvox voxels needs: the chains, then
 // the per-measurement cache rows unless the launch keeps them in LDS.
 size_t mcmc_state_bytes(const cdm_model* m, int nvox, int nmeas, const float* cfp, const float* fixp, int rician) {
   const int L = group_for(m, cdm::kMcmc, nmeas, nvox);
   const cdm::Geom g = make_geom(m, nvox, nmeas, nullptr, cfp, fixp);
-  if (!m->ops->mvc_bytes_per_meas || m->ops->mcmc_rows_lds(L, mcmc_budget(m, nmeas, rician), g))
+  if (!m->ops->mvc_bytes_per_meas || m->ops->mcmc_rows_lds(L, mcmc_budget(m, nmeas, rician, nvox, L), g))
     return m->ops->chain_bytes * (size_t)nvox;
   return mvc_offset(m, nvox) + m->ops->mvc_bytes_per_meas * 2 * (size_t)nmeas * (size_t)nvox;
 }
@@ -914,12 +925,12 @@ int run_mcmc(cdm_model* m, int nvox, int nmeas, const float* meas, float* params
   const cdm::Geom g = make_geom(m, nvox, nmeas, meas, cfp, fixp);
   const cdm::Consts c = make_consts(m);
   const int L = group_for(m, cdm::kMcmc, nmeas, nvox);
-  const int W = occ_for(m, cdm::kMcmc, nmeas);
+  const int W = mcmc_budget(m, nmeas, rician, nvox, L);
 
   cdm::McmcLaunch ml;
   ml.params = params;
   ml.state = state;
-  ml.mvc = (m->ops->mvc_bytes_per_meas && !m->ops->mcmc_rows_lds(L, mcmc_budget(m, nmeas, rician), g))
+  ml.mvc = (m->ops->mvc_bytes_per_meas && !m->ops->mcmc_rows_lds(L, W, g))
                ? (void*)((char*)state + mvc_offset(m, nvox))
                : nullptr;
   ml.samples = samples;
