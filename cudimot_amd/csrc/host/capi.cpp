@@ -183,7 +183,10 @@ constexpr long long kLaneSlots = 256LL * 4 * 64 * 2;
 // 1.3 to 1.6 times the work per voxel (the step's serial part runs on every
 // lane).  NODDI_Bingham, 350 jumps, at 4 and 16 lanes: 32,768 voxels 32.5 and
 // 47.7 ms, 16,384 voxels 22.2 and 24.5, 8,192 voxels 22.2 and 13.0;
-// Ball_2_Sticks 30,000 voxels 27.2 and 28.4, 20,480 voxels 26.4 and 20.5.
+// Ball_2_Sticks 30,000 voxels 27.2 and 28.4, 20,480 voxels 26.4 and 20.5.  The
+// Rician likelihood, whose logarithms and Bessel functions the lanes share, keeps
+// the higher one (26,000 voxels, 30 jumps, 4 and 16 lanes: Ball_2_Sticks 26.8 and 22.8 ms,
+// DiffusionTensor 5.2 and 4.8).
 constexpr long long kMcmcLaneSlots = 256LL * 4 * 64 * 5 / 4;
 
 // Tuned entry of the nearest measurement count (log ratio), or null.
@@ -201,11 +204,11 @@ const cdm_model::Tuned* tuned_for(const cdm_model* m, int method, int nmeas) {
   return best;
 }
 
-int group_for(const cdm_model* m, int method, int nmeas, int nvox) {
+int group_for(const cdm_model* m, int method, int nmeas, int nvox, int rician = 0) {
   if (m->group[method]) return m->group[method];
   const cdm_model::Tuned* t = tuned_for(m, method, nmeas);
   int L = t ? t->lanes : default_group(method, nmeas);
-  const long long floor = method == cdm::kMcmc ? kMcmcLaneSlots : kLaneSlots;
+  const long long floor = method == cdm::kMcmc && !rician ? kMcmcLaneSlots : kLaneSlots;
   while (nvox > 0 && L < 64 && (long long)nvox * L < floor) L *= 4;
   return L;
 }
@@ -904,7 +907,7 @@ int mcmc_budget(const cdm_model* m, int nmeas, int rician, int nvox, int L) {
 // Bytes of chain state an MCMC call over nvox voxels needs: the chains, then
 // the per-measurement cache rows unless the launch keeps them in LDS.
 size_t mcmc_state_bytes(const cdm_model* m, int nvox, int nmeas, const float* cfp, const float* fixp, int rician) {
-  const int L = group_for(m, cdm::kMcmc, nmeas, nvox);
+  const int L = group_for(m, cdm::kMcmc, nmeas, nvox, rician);
   const cdm::Geom g = make_geom(m, nvox, nmeas, nullptr, cfp, fixp);
   if (!m->ops->mvc_bytes_per_meas || m->ops->mcmc_rows_lds(L, mcmc_budget(m, nmeas, rician, nvox, L), g))
     return m->ops->chain_bytes * (size_t)nvox;
@@ -924,7 +927,7 @@ int run_mcmc(cdm_model* m, int nvox, int nmeas, const float* meas, float* params
   const int nsamples = njumps / sampleevery;
   const cdm::Geom g = make_geom(m, nvox, nmeas, meas, cfp, fixp);
   const cdm::Consts c = make_consts(m);
-  const int L = group_for(m, cdm::kMcmc, nmeas, nvox);
+  const int L = group_for(m, cdm::kMcmc, nmeas, nvox, rician);
   const int W = mcmc_budget(m, nmeas, rician, nvox, L);
 
   cdm::McmcLaunch ml;
@@ -1373,7 +1376,7 @@ static int batch_mcmc_persistent(int nitems, const cdm_batch_item* items, int nb
       const cdm_batch_item& it = items[order[k]];
       cdm::BatchLaunchItem& b = li[k];
       b.model = index[order[k]];
-      b.L = group_for(it.model, cdm::kMcmc, it.nmeas, (int)std::min<long long>(total, INT_MAX));
+      b.L = group_for(it.model, cdm::kMcmc, it.nmeas, (int)std::min<long long>(total, INT_MAX), rician);
       b.g = make_geom(it.model, it.nvox, it.nmeas, it.meas, it.cfp, it.fixp);
       b.c = make_consts(it.model);
       b.params = it.params;

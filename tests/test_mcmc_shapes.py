@@ -46,3 +46,15 @@ def test_small_volumes_take_the_registers_they_can_have(model, n):
         by_hand.append(_ms(go))
         assert (s == first).all()
     assert own < 1.12 * min(by_hand) + 0.03, (own, by_hand)
+
+
+@pytest.mark.parametrize("n", [21000, 26000])
+def test_rician_chains_of_mid_size_volumes_take_the_better_lanes(n):
+    from cudimot_amd import capi
+    m, go, _ = _calls("Ball_2_Sticks", n, True, 15)
+    own = _ms(go)
+    by_hand = []
+    for lanes in (4, 16):
+        m.set_group(capi.MCMC, lanes)
+        by_hand.append(_ms(go))
+    assert own < 1.08 * min(by_hand), (own, by_hand)
