@@ -3123,14 +3123,19 @@ struct cdm_post_args {
 };
 
 // The mean samples of the block's voxels, handed to each voxel's lanes in mp
-// (and the mean tau, with tau_samples): 16 lanes per row of samples, so that a
-// wave reads runs of adjacent values (a thread per row below 16 samples, where
-// adjacent rows are near enough and 16 rows at a time are too few), into the dynamic LDS before anything else
-// is staged there.  Every lane of a voxel reading all of its samples by itself
-// took most of these kernels (NODDI_Bingham, 200k voxels, 50 samples, 99
-// measurements: predicted signal 0.48 -> 0.20 ms, BIC/AIC 0.54 -> 0.28 ms).
+// (and the mean tau, with tau_samples), into the dynamic LDS before anything else
+// is staged there: 16 lanes per row of samples, so that a wave reads runs of
+// adjacent values, or a thread per row of few samples, where adjacent rows are near
+// enough and 16 rows at a time are too few.  Every lane of a voxel reading all of
+// its samples by itself took most of these kernels (NODDI_Bingham, 200k voxels, 50
+// samples, 99 measurements: predicted signal 0.48 -> 0.20 ms, BIC/AIC 0.54 -> 0.28 ms).
+// The line lies higher for the plug-ins with a voxel cache, whose kernels have fewer
+// waves to hide a row's latency: 200k voxels, 16 samples, BIC/AIC by 16 lanes and by
+// threads NODDI_Bingham_2Fans 382 and 262 us, NODDI_Bingham 151 and 128,
+// Ball_2_Sticks 116 and 136, DiffusionTensor 67 and 82; 20 samples NODDI_Bingham's
+// signal 142 and 190.
 // Ends with a barrier; every thread of the block takes part.
-constexpr int cdm_mean_lanes = 16;
+constexpr int cdm_mean_lanes = 16, cdm_mean_few = cdm_vc > 1 ? 18 : 16;
 template <int L>
 __device__ __forceinline__ void cdm_mean_samples(const cdm_post_args& a, double* s_mean, bool rician, double* mp,
                                                  double* tau) {
@@ -3141,7 +3146,7 @@ __device__ __forceinline__ void cdm_mean_samples(const cdm_post_args& a, double*
   auto row = [&](int q, int i) {
     return i < cdm_np ? a.samples + ((size_t)(v0 + q) * cdm_np + i) * S : a.tau_samples + (size_t)(v0 + q) * S;
   };
-  if (S < cdm_mean_lanes) {
+  if (S < cdm_mean_few) {
     for (int r = threadIdx.x; r < nv * width; r += cdm_block) {
       const int q = r / width, i = r - q * width;
       const float* s = row(q, i);
