@@ -1402,10 +1402,13 @@ __device__ __forceinline__ double cdm_dtransform1(int bt, float lo, float hi, do
 // The transforms of all parameters by a group of L lanes: lane i (i + L, ...)
 // transforms parameter i and hands it to the group, so the exponentials and
 // arctangents of all parameters issue once instead of one after the other.  One
-// lane per voxel does them in turn, and so do the batch units, whose kernels
-// run out of registers already (the spread form compiled there to a kernel that
-// rejected every step of the 14-parameter plug-in).  Same values either way.
-// DiffusionTensor, the same kernel otherwise: 1.27 -> 0.99 ms.
+// lane per voxel does them in turn, and so do the batch units: there the spread
+// form meets the compiler's fault that the build looks for (copies of the base
+// point's 1F1 values before a mask update in the 64-lane fit of
+// NODDI_Bingham_2Fans, which then rejects its steps).  Same values either way,
+// compared for the nine plug-ins at every group size and register budget.
+// Serial over spread times, 3,000 voxels at 4 iterations: DiffusionTensor 1.34,
+// Ball_3_Sticks 1.20, NODDI_Watson 1.38, NODDI_Bingham_2Fans 1.74.
 #ifdef CDM_BATCH_UNIT
 constexpr bool cdm_lane_transforms = false;
 #else
