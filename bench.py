@@ -68,9 +68,10 @@ PEAK_F32 = 157.3e12
 # readings for a 512 MiB copy (fetch x2.0, write x1.0):
 # - per voxel and launch: the measurements read, the chain state and
 #   parameters written (721 B);
-# - per voxel and jump: 32 bytes of scratch per lane that the steps in an angle
-#   write (burn-in launch: 309,283 + 3,003,687 KiB / 131,072 voxels, less the
-#   721 B, over 100 jumps);
+# - per voxel and jump: what reaches HBM of the 32 bytes of scratch per lane that
+#   each step in an angle writes (4 lanes and 3 angles a voxel, 384 B at most;
+#   burn-in launch: 309,283 + 3,003,687 KiB / 131,072 voxels, less the 721 B,
+#   over 100 jumps);
 # - per stored sample value: one 32-byte sector and more, since a launch stores
 #   one sample of each parameter per recording and a parameter's samples lie
 #   contiguous per voxel ((30,659 + 331,689) KiB / 9,175,040 stores).
@@ -506,7 +507,7 @@ def main():
                                           P * nsamp * MCMC_BYTES_PER_SAMPLE_STORE) / 2,
                 "traffic_note": "HBM bytes per launch (mean of the burn-in and recording launches) from rocprofv3 "
                                 "FETCH_SIZE/WRITE_SIZE, copy-calibrated: measurements and chain state per voxel, "
-                                "32 bytes of scratch per lane written by the steps in an angle, a sector per "
+                                "scratch written by the steps in an angle (252 B per voxel and jump), a sector per "
                                 "stored sample; the cache rows stay in LDS: 0.1 TB/s, so the kernel is bound by "
                                 "vector-ALU issue, not HBM",
                 "flops_per_launch_f32": f32 / 2, "flops_per_launch_f64": f64 / 2,

@@ -11,10 +11,11 @@ operation-counting scalar (lib/libcdm_opcount.so, csrc/tools/opcount.h):
 +, -, * = 1, / and sqrt = 1, each transcendental = 1, FMA = 2.  Method
 totals per voxel:
   MCMC  = jumps * sum_params M * (F_meas + 3 FP32 + 1 FP64)  (residual,
-          square, FP64 accumulation per measurement; F_meas is the cached
-          per-measurement signal, plus the per-measurement cache when the
-          proposed parameter is one it depends on; proposals and priors are
-          O(P) per jump and not counted) + voxel caches of dependent proposals
+          square, FP64 accumulation per measurement; F_meas is the signal from
+          the kept per-measurement values, or with those formed anew when the
+          proposed parameter moves them, and from the kept frame; proposals and
+          priors are O(P) per jump and not counted) + voxel caches and frames
+          of the proposals that move them
   LM    = sum over iterations of M * (F_fwd + F_jac + P(P+1)/2 * 2 + 2P)
           for accepted steps plus M * F_fwd per cost evaluation
   GS    = combinations * M * (F_fwd + 3)
@@ -44,7 +45,7 @@ def per_eval(model, params, cfp, fixp=None):
     cfp = np.ascontiguousarray(cfp, dtype=np.float64)
     n = params.shape[0]
     fixp = np.ascontiguousarray(fixp if fixp is not None else np.zeros((n, 1)), dtype=np.float64)
-    out = np.zeros(20)
+    out = np.zeros(27)
     D = ctypes.POINTER(ctypes.c_double)
     getattr(_load(), "cdm_opcount_" + model)(n, cfp.shape[0], params.ctypes.data_as(D), cfp.ctypes.data_as(D),
                                              fixp.ctypes.data_as(D), out.ctypes.data_as(D))
@@ -53,26 +54,23 @@ def per_eval(model, params, cfp, fixp=None):
             "vc32": out[8], "vc64": out[9], "vc_dep": int(out[10]), "cached": bool(out[11]),
             "meas32": out[12], "meas64": out[13],
             "mv32": out[14], "mv64": out[15], "pmv32": out[16], "pmv64": out[17], "mvc_dep": int(out[18]),
-            "mvc": bool(out[19])}
+            "mvc": bool(out[19]), "kept32": out[20], "kept64": out[21], "moved32": out[22], "moved64": out[23],
+            "fr_dep": int(out[24]), "fr32": out[25], "fr64": out[26]}
 
 
 def mcmc_flops(ev, nparams, nmeas, jumps):
     """(FP32, FP64) flops of one voxel's MCMC over `jumps` jumps: every
     proposal evaluates the signal at all measurements, recomputes the voxel
-    cache when the proposed parameter is one it depends on, and (with
-    per-measurement caches) recomputes those only when it depends on them."""
+    cache, its parameter's run of the frame and (with per-measurement caches)
+    those when the proposed parameter is one they depend on."""
     ndep = bin(ev["vc_dep"]).count("1") if ev["cached"] else 0
-    f32 = jumps * ndep * ev["vc32"]
-    f64 = jumps * ndep * ev["vc64"]
+    nfr = bin(ev["fr_dep"]).count("1")
+    f32 = jumps * (ndep * ev["vc32"] + nfr * ev["fr32"])
+    f64 = jumps * (ndep * ev["vc64"] + nfr * ev["fr64"])
     for i in range(nparams):
-        if ev.get("mvc"):
-            dep = (ev["mvc_dep"] >> i) & 1
-            m32 = ev["pmv32"] + (ev["mv32"] if dep else 0.0)
-            m64 = ev["pmv64"] + (ev["mv64"] if dep else 0.0)
-        else:
-            m32, m64 = ev["meas32"], ev["meas64"]
-        f32 += jumps * nmeas * (m32 + 3)
-        f64 += jumps * nmeas * (m64 + 1)
+        form = "moved" if (ev["mvc_dep"] >> i) & 1 else "kept"
+        f32 += jumps * nmeas * (ev[form + "32"] + 3)
+        f64 += jumps * nmeas * (ev[form + "64"] + 1)
     return f32, f64
 
 

@@ -26,3 +26,20 @@ def test_bingham_mcmc_flops_use_the_per_measurement_cache():
     ev = flops.per_eval("NODDI_Bingham", synth.truth_for("NODDI_Bingham", 6, 2), cfp, np.full((6, 1), 1000.0))
     assert ev["mvc"] and ev["mvc_dep"] == 0x7C
     assert ev["mv64"] > 0 and ev["pmv64"] == 0
+
+
+@pytest.mark.parametrize("model", ["Ball_1_Stick", "Ball_2_Sticks", "Ball_3_Sticks", "NODDI_Watson", "NODDI_Bingham"])
+def test_kept_frames_leave_no_sines_in_a_measurement(model):
+    """A chain takes the sine and cosine of an angle once per step that moves it,
+    not at every measurement."""
+    from cudimot_amd import flops, synth
+    cfp = synth.model_acquisition(model)
+    ev = flops.per_eval(model, synth.truth_for(model, 6, 2), cfp, np.full((6, 1), 1000.0))
+    angles = bin(ev["fr_dep"]).count("1")
+    assert angles >= 2 and ev["fr32"] + ev["fr64"] == 2
+    whole = ev["pmv32"] + ev["mv32"] if ev["mvc"] else ev["meas32"]
+    assert ev["moved32"] <= whole - 2 * angles and ev["kept32"] <= ev["moved32"]
+    f32, f64 = flops.mcmc_flops(ev, 1, 10, 3)
+    vc = bin(ev["vc_dep"]).count("1")
+    assert f32 == pytest.approx(3 * (vc * ev["vc32"] + angles * ev["fr32"] + 10 * (ev["kept32"] + 3)))
+    assert f64 == pytest.approx(3 * (vc * ev["vc64"] + angles * ev["fr64"] + 10 * (ev["kept64"] + 1)))
