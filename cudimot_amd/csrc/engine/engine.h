@@ -873,9 +873,11 @@ __global__ void __launch_bounds__(cdm_block) cdm_gridsearch_pick_kernel(cdm_gs_a
 // need two butterfly stages, and the combinations of the weight parameters are
 // spread over the lanes.
 //
-// Bound by VALU issue: about 18 slots per measurement and basis combination
-// (one exponential, the FP64 products).  Measured against the scan of every
-// combination: NODDI_Watson, 968 combinations, 99 measurements, 150k voxels
+// Bound by the latency of LDS reads at low occupancy: about 18 issue slots per
+// measurement and basis combination (one exponential, the FP64 products), but 60
+// measured, since a block's rows (94 KB NODDI_Watson, 110 KB NODDI_Bingham, 65 KB
+// Ball_2_Sticks at 16 lanes) leave one or two blocks per CU, a wave per SIMD each.
+// Measured against the scan of every combination: NODDI_Watson, 968 combinations, 99 measurements, 150k voxels
 // 90.1 -> 2.05 ms; Ball_2_Sticks, 729 combinations, 280 measurements, 50k voxels
 // 25.1 -> 1.45 ms; NODDI_Bingham, 11,050 combinations, 307 voxels 12.3 ->
 // 0.33 ms (the screen in 154 slices).  One loop over a row of adjacent values

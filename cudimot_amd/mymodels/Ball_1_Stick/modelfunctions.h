@@ -33,7 +33,7 @@ MACRO T Predicted_Signal(int npar, T* P, T* CFP, T* FixP) {
   return P[0] * (((T)1 - P[2]) * ball + P[2] * stick);
 }
 
-// MCMC hooks: the signal from the sines and cosines of the sticks' angles.
+// MCMC hooks: the signal from the sines and cosines of the stick's angles.
 #define CDM_SIGNAL_FRAME 4
 #define CDM_SIGNAL_FRAME_DEPENDS 0x18u
 
@@ -61,8 +61,8 @@ MACRO T Predicted_Signal_Framed(int npar, T* P, T* CFP, T* FixP, const double* v
   return P[0] * (((T)1 - P[2]) * ball + P[2] * stick);
 }
 
-// GridSearch hooks: the signal is linear in the fractions and S0; the ball
-// are shared by the combinations of the last stick's angles.
+// GridSearch hooks: the signal is linear in the fraction and S0; the ball is
+// shared by the combinations of the stick's angles.
 #define CDM_GRID_LINEAR 0x05u        // S0, f
 #define CDM_GRID_SHARED 0x02u        // d
 #define CDM_GRID_SHARED_VALUES 1

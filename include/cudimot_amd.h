@@ -117,7 +117,8 @@ int cdm_model_graph_stats(const cdm_model* m, long long* captures, long long* re
  * device int[nvox]) receives the kept combination index, -1 if none.
  * Plug-ins with GridSearch basis hooks (the shipped stick and NODDI models but
  * NODDI_Bingham_2Fans) evaluate what combinations share once; other plug-ins,
- * and calls under stream capture, scan every combination.  Volumes too small
+ * grids whose combinations share little, and calls under stream capture, scan
+ * every combination.  Volumes too small
  * to fill the GPU search slices of the combinations in parallel.  The result is
  * the same either way.  Scratch is allocated on the handle at the first call
  * of a larger size (the scan of a volume that fills the GPU needs none). */
