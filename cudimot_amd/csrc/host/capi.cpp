@@ -184,9 +184,10 @@ constexpr long long kLaneSlots = 256LL * 4 * 64 * 2;
 // lane).  NODDI_Bingham, 350 jumps, at 4 and 16 lanes: 32,768 voxels 32.5 and
 // 47.7 ms, 16,384 voxels 22.2 and 24.5, 8,192 voxels 22.2 and 13.0;
 // Ball_2_Sticks 30,000 voxels 27.2 and 28.4, 20,480 voxels 26.4 and 20.5.  The
-// Rician likelihood, whose logarithms and Bessel functions the lanes share, keeps
-// the higher one (26,000 voxels, 30 jumps, 4 and 16 lanes: Ball_2_Sticks 26.8 and 22.8 ms,
-// DiffusionTensor 5.2 and 4.8).
+// Rician likelihood, whose logarithms and Bessel functions the lanes share, widens
+// from 4 lanes by the higher one (26,000 voxels, 30 jumps, 4 and 16 lanes:
+// Ball_2_Sticks 26.8 and 22.8 ms, DiffusionTensor 5.2 and 4.8), but not from 16: 64
+// lanes take 1.2 to 1.9 times as long at 7,000 voxels (1.0 for 280 measurements).
 constexpr long long kMcmcLaneSlots = 256LL * 4 * 64 * 5 / 4;
 
 // Tuned entry of the nearest measurement count (log ratio), or null.
@@ -208,8 +209,8 @@ int group_for(const cdm_model* m, int method, int nmeas, int nvox, int rician = 
   if (m->group[method]) return m->group[method];
   const cdm_model::Tuned* t = tuned_for(m, method, nmeas);
   int L = t ? t->lanes : default_group(method, nmeas);
-  const long long floor = method == cdm::kMcmc && !rician ? kMcmcLaneSlots : kLaneSlots;
-  while (nvox > 0 && L < 64 && (long long)nvox * L < floor) L *= 4;
+  auto floor = [&] { return method == cdm::kMcmc && !(rician && L < 16) ? kMcmcLaneSlots : kLaneSlots; };
+  while (nvox > 0 && L < 64 && (long long)nvox * L < floor()) L *= 4;
   return L;
 }
 

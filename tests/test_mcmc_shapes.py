@@ -58,3 +58,16 @@ def test_rician_chains_of_mid_size_volumes_take_the_better_lanes(n):
         m.set_group(capi.MCMC, lanes)
         by_hand.append(_ms(go))
     assert own < 1.08 * min(by_hand), (own, by_hand)
+
+
+@pytest.mark.parametrize("model", ["NODDI_Watson", "Ball_1_Stick"])
+@pytest.mark.parametrize("n", [5600, 7000])
+def test_rician_chains_of_small_volumes_keep_16_lanes(model, n):
+    from cudimot_amd import capi
+    m, go, _ = _calls(model, n, True, 48)
+    own = _ms(go)
+    by_hand = []
+    for lanes in (16, 64):
+        m.set_group(capi.MCMC, lanes)
+        by_hand.append(_ms(go))
+    assert own < 1.08 * min(by_hand), (own, by_hand)
