@@ -258,12 +258,17 @@ static hipError_t op_levmar(int L, int W, const cdm::Geom& g, float* params, int
 // jumps 28.1 and 43.8 ms, 14k (1.7) 18.7 and 21.4; Ball_1_Stick, 66k (1.01), 300 jumps
 // 8.7 and 11.1, but 300k (4.6), 64 jumps 8.6 and 7.3; toymodel, 66k, 300 jumps 3.1 and
 // 2.6; DiffusionTensor, 300k, 64 jumps 9.8 and 9.0.
+//   Rician launches, whose terms are dear and differ in time, take all of them: 4,000
+// voxels, 100 jumps, with and without, Ball_2_Sticks 25.5 and 28.8 ms, NODDI_Bingham
+// 14.1 and 15.7, DiffusionTensor 7.0 and 7.4; 3,300 and 40 jumps 9.4 and 11.3, 5.2 and
+// 5.2, 2.6 and 3.0; 140k and 100 jumps, Ball_1_Stick 103.5 and 108.1.
 constexpr int cdm_mcmc_rounds = 16, cdm_mcmc_least_jumps = 16;
-static int op_mcmc_slices(int tiles, int per_cu, int ncu, int count, int nmeas, int L) {
+static int op_mcmc_slices(int tiles, int per_cu, int ncu, int count, int nmeas, int L, bool rician) {
   const long long R = (long long)per_cu * ncu;
   if (R <= 0 || tiles <= R) return 1;
   const long long want = (cdm_mcmc_rounds * R + tiles - 1) / tiles;
   const int most = (int)std::min<long long>(want, count / cdm_mcmc_least_jumps);
+  if (rician) return most > 1 ? most : 1;
   const double r = (double)tiles / R, whole = (double)((tiles + R - 1) / R);
   const double terms = (double)count * cdm_np * ((nmeas + L - 1) / L * (cdm_vc > 1 ? 8 : 1) + 3);
   int n = 1;
@@ -287,7 +292,7 @@ static hipError_t op_mcmc_launch(cdm_mcmc_args a, size_t lds, int* queue, int nc
     const hipError_t e =
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (cdm_mcmc_kernel<L, RICIAN, W>), cdm_block, lds);
     if (e != hipSuccess) return e;
-    const int n = op_mcmc_slices(a.ntiles, per_cu, ncu, a.count, a.g.nmeas, L);
+    const int n = op_mcmc_slices(a.ntiles, per_cu, ncu, a.count, a.g.nmeas, L, RICIAN);
     if (n > 1) {
       a.queue = queue;
       a.chunk_len = (a.count + n - 1) / n;

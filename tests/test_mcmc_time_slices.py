@@ -135,3 +135,38 @@ def test_light_models_take_one_block_per_tile(model, n, jumps):
     go(None)
     tiles = (n * m.get_group(capi.MCMC, cfp.shape[0], n) + 255) // 256
     assert _grids(go) == [tiles, tiles]
+
+
+@pytest.mark.parametrize("model,n,jumps", [("Ball_2_Sticks", 4000, 100), ("DiffusionTensor", 3300, 40)])
+def test_rician_launches_of_few_rounds_take_slices(model, n, jumps):
+    """No slower than the chains without slices, and the same."""
+    import torch
+    from cudimot_amd import capi
+    m, t, cfp, fixp, meas = _volume(model, n)
+    m.set_group(capi.MCMC, 64)
+    s = torch.empty((n, m.nparams, 1), device="cuda")
+    tau = torch.empty((n, 1), device="cuda")
+    p = t.clone()
+
+    def go(f, a, b, q=None):
+        p.copy_(t)
+        f(meas[a:b], p[a:b], cfp, None if fixp is None else fixp[a:b], s[a:b], tau[a:b], nburn=jumps, njumps=jumps,
+          sampleevery=jumps, rician=True, seed=5, voxel_offset=a, stream=q or torch.cuda.current_stream())
+
+    def ms(f):
+        best = float("inf")
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            f()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+    go(m.mcmc, 0, n)
+    assert min(_grids(lambda q: go(m.mcmc, 0, n, q))) >= 2 * n // 4
+    sliced = ms(lambda: go(m.mcmc, 0, n))
+    got = s.clone(), tau.clone()
+    whole = ms(lambda: [go(m.mcmc_noalloc, a, min(n, a + 1500)) for a in range(0, n, 1500)])
+    assert torch.equal(got[0], s) and torch.equal(got[1], tau)
+    assert sliced < whole, (sliced, whole)
