@@ -253,11 +253,13 @@ static hipError_t op_levmar(int L, int W, const cdm::Geom& g, float* params, int
 // r = tiles / resident and ceil(n r) / n rounds, and each a hand-over (the chain
 // state through memory, an L2 write-back, the prologue) worth 250 likelihood terms of
 // a lane.  A step has ceil(M / L) terms, eight times the cost for plug-ins with a
-// voxel cache, and draws worth three.  At most as many slices as fill sixteen rounds, of
+// voxel cache, and draws worth three (with 64 lanes and their sums twelve).  At most as many slices as fill sixteen rounds, of
 // 16 jumps at least.  Measured with and without: NODDI_Bingham, 35k voxels (r = 1.07), 300
 // jumps 28.1 and 43.8 ms, 14k (1.7) 18.7 and 21.4; Ball_1_Stick, 66k (1.01), 300 jumps
 // 8.7 and 11.1, but 300k (4.6), 64 jumps 8.6 and 7.3; toymodel, 66k, 300 jumps 3.1 and
 // 2.6; DiffusionTensor, 300k, 64 jumps 9.8 and 9.0.
+//   With 64 lanes, 70 jumps, 4,153 voxels (r = 2.0), with and without, DiffusionTensor 2.2
+// and 2.7, Ball_1_Stick 2.0 and 2.3; 32 jumps, NODDI_Watson 3.3 and 3.7.
 //   Rician launches, whose terms are dear and differ in time, take all of them: 4,000
 // voxels, 100 jumps, with and without, Ball_2_Sticks 25.5 and 28.8 ms, NODDI_Bingham
 // 14.1 and 15.7, DiffusionTensor 7.0 and 7.4; 3,300 and 40 jumps 9.4 and 11.3, 5.2 and
@@ -270,7 +272,7 @@ static int op_mcmc_slices(int tiles, int per_cu, int ncu, int count, int nmeas, 
   const int most = (int)std::min<long long>(want, count / cdm_mcmc_least_jumps);
   if (rician) return most > 1 ? most : 1;
   const double r = (double)tiles / R, whole = (double)((tiles + R - 1) / R);
-  const double terms = (double)count * cdm_np * ((nmeas + L - 1) / L * (cdm_vc > 1 ? 8 : 1) + 3);
+  const double terms = (double)count * cdm_np * ((nmeas + L - 1) / L * (cdm_vc > 1 ? 8 : 1) + (L == 64 ? 12 : 3));
   int n = 1;
   double best = per_cu > 2 ? r + 0.4 * (whole - r) : whole;
   for (int k = 2; k <= most; ++k) {

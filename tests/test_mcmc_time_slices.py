@@ -170,3 +170,18 @@ def test_rician_launches_of_few_rounds_take_slices(model, n, jumps):
     whole = ms(lambda: [go(m.mcmc_noalloc, a, min(n, a + 1500)) for a in range(0, n, 1500)])
     assert torch.equal(got[0], s) and torch.equal(got[1], tau)
     assert sliced < whole, (sliced, whole)
+
+
+@pytest.mark.parametrize("model,n,jumps", [("DiffusionTensor", 4153, 70), ("NODDI_Watson", 4153, 32), ("Ball_1_Stick", 4313, 70)])
+def test_short_chains_at_64_lanes_take_slices(model, n, jumps):
+    """Launches of two rounds and a little more, whose last is nearly empty."""
+    import torch
+    from cudimot_amd import capi
+    m, t, cfp, fixp, meas = _volume(model, n)
+    m.set_group(capi.MCMC, 64)
+    s = torch.empty((n, m.nparams, 1), device="cuda")
+    p = t.clone()
+    go = lambda q: m.mcmc(meas, p, cfp, fixp, s, nburn=jumps, njumps=jumps, sampleevery=jumps, stream=q)  # noqa: E731
+    go(None)
+    torch.cuda.synchronize()
+    assert min(_grids(go)) >= 2 * ((n + 3) // 4)
